@@ -20,7 +20,7 @@ ROCM = pathlib.Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 HIPCC = ROCM / "bin" / "hipcc"
 
 FLAGS = [
-    "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-mcode-object-version=5",
+    "-O3", "-std=c++20", "-fPIC", "--offload-arch=gfx950", "-mcode-object-version=5",
     # packed fp32 instructions stay off: hipcc would otherwise form them from float code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",

@@ -15,7 +15,8 @@
 // (DPP), a row (DPP rotate / mirror) and the wave (shuffles). Many rows (a prompt) run on the matrix cores: int8 and
 // the codes on the int8 cores against the rows as three int8 planes with a power-of-two scale (grouped_i8_kernel),
 // FP8 on the bf16 cores against exact bf16 planes (grouped_fp8_kernel), each weight read once per 32-row pass.
-#include "common.hpp"
+#include "ref_common.hpp"
+#include "wide_tile.hpp"
 #include "../../include/drama3_moe.h"
 
 #include <algorithm>
@@ -26,10 +27,6 @@ int fail(const std::string& msg);
 int hip_fail(hipError_t err, const char* what);
 
 constexpr int RPB = 16;  // output rows per workgroup of the GEMVs (kernels.py:590 ROWS_PER_BLOCK: N % 16 == 0)
-
-template <int CTRL> D3_INLINE float dpp_f32(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
 
 // ---------------------------------------------------------------------------------------------------------- route
 // kernels.py:39-67: the k (<= 32) largest of n (<= 1024) bf16 logits, descending, ties to the lower index; weights
@@ -282,37 +279,6 @@ D3_INLINE void decode_group(uint32_t lo, uint32_t hi, uint32_t high, uint32_t sc
     else value = lut[code];
     q[j] = fminf(fmaxf(rintf(value * s), -127.0f), 127.0f);
   }
-}
-
-// W4 through tables: a 16-column group's codes all share one e4m3 scale byte, so the int8-grid values of the 16 codes at
-// each of the 256 scale bytes make a 4 KB table (decode_group's own arithmetic, entry by entry), kept in LDS as bytes
-// q + 128. A group then costs one 16-byte table read, and four of its codes become four bytes through two byte
-// permutes and a byte mask, instead of a codebook read, a product, a rounding and a clamp per value.
-constexpr int QTAB_WORDS = 256 * 4;  // qtab[4 sb + i]: bytes q + 128 of codes 4i .. 4i + 3 at scale byte sb
-// cb: codebook[4 (threadIdx.x & 3) .. + 3], loaded by the caller (ahead of its weight rows); SIGNED: the bytes hold q
-// itself (two's complement) instead of q + 128
-template <bool SIGNED = false> D3_INLINE void build_qtab(uint32_t* qtab, f32x4 cb) {
-  const float c[4] = {cb.x, cb.y, cb.z, cb.w};
-  for (int i = threadIdx.x; i < QTAB_WORDS; i += blockDim.x) {  // i & 3 == threadIdx.x & 3: blockDim.x % 4 == 0
-    const float sc = fp8x2_to_f32<false>((uint32_t)(i >> 2)).x;
-    uint32_t word = 0u;
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-      const float q = fminf(fmaxf(rintf(c[b] * sc), -127.0f), 127.0f);
-      word |= ((uint32_t)((int)q + (SIGNED ? 0 : 128)) & 0xFFu) << (8 * b);
-    }
-    qtab[i] = word;
-  }
-}
-
-// the table bytes (t: entries 0..15, 4 per word) at the four indices held in the low nibbles of sel's bytes
-D3_INLINE uint32_t lookup16(i32x4 t, uint32_t sel) {
-  const uint32_t s3 = sel & 0x07070707u;
-  const uint32_t lo = __builtin_amdgcn_perm((uint32_t)t.y, (uint32_t)t.x, s3);  // entries 0..7
-  const uint32_t hi = __builtin_amdgcn_perm((uint32_t)t.w, (uint32_t)t.z, s3);  // entries 8..15
-  // selector byte 12 gives 0x00, 13 gives 0xFF: a byte mask of the indices >= 8
-  const uint32_t m = __builtin_amdgcn_perm(0u, 0u, ((sel >> 3) & 0x01010101u) | 0x0C0C0C0Cu);
-  return (hi & m) | (lo & ~m);
 }
 
 // sum over one group of (q + 128) * x for its 16 codes (nibble words lo / hi, table row t), x the group's 16 floats
@@ -620,9 +586,12 @@ __global__ void __launch_bounds__(256) grouped_plan_kernel(const int* groups, in
 // after every group, inverse -1. With `work`, the same workgroup also plans the grouped products' passes over the
 // groups (grouped_plan_kernel's plan, from the counts it holds), so that takes no launch of its own.
 constexpr int GROUPS_MAX_E = 1024;
+// With `wide`, the passes of the wide products instead (pass_cap places of (expert, first row, rows, 0) after the count
+// at wide[0], at most WIDE_TILES 16-row tiles each): the passes with most tiles first, an expert's passes together.
 D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* order, int* inverse, int* groups,
-                                  int* work, int cap) {
+                                  int* work, int cap, int* wide, int wide_cap) {
   __shared__ int count[GROUPS_MAX_E + 1], cursor[GROUPS_MAX_E + 1], wave_total[16], pcount[8], pcursor[8];
+  static_assert(WIDE_TILES <= 8, "a bucket of pcount per number of tiles");
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int e = tid; e <= E; e += 1024) count[e] = 0;
   if (tid < 8) pcount[tid] = 0;
@@ -646,7 +615,7 @@ D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* ord
   for (int i = 0; i < w; i++) before += wave_total[i];
   const int first = before + incl - v;
   if (tid <= E) cursor[tid] = first;
-  if (tid < E) {
+  if (groups && tid < E) {
     int* gp = groups + 5 * tid;
     gp[0] = tid;
     gp[1] = tid;
@@ -666,6 +635,25 @@ D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* ord
     __syncthreads();
     if (tid < E) plan_put(tid, first, v, P, pcursor, work, cap);
   }
+  if (wide) {  // bucket b: passes of WIDE_TILES - b tiles
+    const int np = tid < E ? wt_passes(v, WIDE_TILES) : 0, tiles = wt_tiles(v, WIDE_TILES);
+    if (np) atomicAdd(&pcount[WIDE_TILES - tiles], np);
+    __syncthreads();
+    if (tid == 0) {
+      int at = 0;
+      for (int b = 0; b < WIDE_TILES; b++) {
+        pcursor[b] = at;
+        at += pcount[b];
+      }
+      wide[0] = min(at, wide_cap);
+    }
+    __syncthreads();
+    if (np) {
+      const int at = atomicAdd(&pcursor[WIDE_TILES - tiles], np), step = 16 * tiles;
+      for (int i = 0; i < np && at + i < wide_cap; i++)
+        ((int4*)(wide + 4))[at + i] = int4{tid, first + i * step, min(step, v - i * step), 0};
+    }
+  }
   __syncthreads();
   for (int p = tid; p < P; p += 1024) {
     const int64_t e = ids[p];
@@ -678,7 +666,7 @@ D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* ord
 
 __global__ void __launch_bounds__(1024) expert_groups_kernel(const int64_t* ids, int P, int E, int64_t* order,
                                                              int* inverse, int* groups, int* work, int cap) {
-  expert_groups_body(ids, P, E, order, inverse, groups, work, cap);
+  expert_groups_body(ids, P, E, order, inverse, groups, work, cap, nullptr, 0);
 }
 
 // columns c0 .. c0 + 3 of row `row` of x as float (SRC as for prep_planes_kernel)
@@ -737,8 +725,6 @@ __global__ void __launch_bounds__(256) prep_planes_kernel(const void* x, const i
 // difference from the exact product, rounded once). So the planes hold v to within (0.5 / 254^2 + 2^-24) S <
 // 1.25e-7 max |v|, and a row of integers times a power of two (such as a one-hot row) exactly in a0. An all-zero row
 // gets S = 0, a row holding a non-finite value S = NaN (planes 0 both ways); below 2^-143, S stays 2^-149.
-constexpr float I8_RATIO = 254.0f;  // the int8 planes' ratio
-
 // Row p of the planes by the row's 4 waves (w = 0 .. 3 of them, lane within the wave, tid0: the row's first thread;
 // wmax: 4 LDS words of the row); valid false: a row past the planes' end, which only joins the barrier. Every
 // thread of the workgroup takes the one barrier inside.
@@ -809,10 +795,10 @@ __global__ void __launch_bounds__(256) prep_i8_kernel(const void* x, const int64
 template <int SRC, bool ROT>
 __global__ void __launch_bounds__(1024) groups_prep_kernel(const int64_t* ids, int P, int E, int64_t* order,
                                                            int* inverse, int* groups, int* work, int cap,
-                                                           const void* x, int T, int K, int8_t* planes,
-                                                           float* scales) {
+                                                           int* wide, int wide_cap, const void* x, int T, int K,
+                                                           int8_t* planes, float* scales) {
   if (blockIdx.x == 0) {
-    expert_groups_body(ids, P, E, order, inverse, groups, work, cap);
+    expert_groups_body(ids, P, E, order, inverse, groups, work, cap, wide, wide_cap);
     return;
   }
   __shared__ uint32_t wmax[4][4];
@@ -868,12 +854,6 @@ D3_INLINE bf16x8 fp8x8_to_bf16(uint32_t w0, uint32_t w1) {
   a[0] = (__bf16)p0.x; a[1] = (__bf16)p0.y; a[2] = (__bf16)p1.x; a[3] = (__bf16)p1.y;
   a[4] = (__bf16)p2.x; a[5] = (__bf16)p2.y; a[6] = (__bf16)p3.x; a[7] = (__bf16)p3.y;
   return a;
-}
-
-// The row of the planes that row p of the passes reads: p itself, or with `order` x's row order[p] / k (the rows of
-// a prompt's pairs taken from its token rows, so no gathered copy is made), kept within the planes' xrows rows.
-D3_INLINE size_t plane_row(const int64_t* order, int k, int xrows, int p) {
-  return order ? (size_t)min(max((int)order[p], 0) / k, xrows - 1) : (size_t)p;
 }
 
 // The fp8 grouped products on the bf16 matrix cores, over PL bf16 planes of the rows (1: bf16 rows as they are).
@@ -1033,16 +1013,6 @@ __global__ void __launch_bounds__(256, 2) grouped_fp8_kernel(const __bf16* xs, i
 // epilogue adds the planes in float32: out = es * (S * (A0 + (A1 + A2 / 254) / 254)). The work list, placement,
 // slot fill and weight ring are grouped_fp8_kernel's; lane group q takes columns 32 q .. 32 q + 31 of each
 // 128-column chunk in 2 steps of 16 bytes, weights and rows alike.
-
-// W4: one 16-code group's int8-grid values as bytes in column order (word d: codes 4d .. 4d + 3) through the
-// group's scale-byte row t of a signed table (build_qtab<true>); lo / hi: the nibble words of codes 0-7 / 8-15
-// (code j's nibble at bits 4 (j & 7))
-D3_INLINE i32x4 w4_group_i8(uint32_t lo, uint32_t hi, i32x4 t) {
-  const uint32_t e0 = lookup16(t, lo), o0 = lookup16(t, lo >> 4);  // codes 0, 2, 4, 6 / 1, 3, 5, 7
-  const uint32_t e1 = lookup16(t, hi), o1 = lookup16(t, hi >> 4);  // codes 8, 10, 12, 14 / 9, 11, 13, 15
-  return i32x4{(int)__builtin_amdgcn_perm(o0, e0, 0x05010400u), (int)__builtin_amdgcn_perm(o0, e0, 0x07030602u),
-               (int)__builtin_amdgcn_perm(o1, e1, 0x05010400u), (int)__builtin_amdgcn_perm(o1, e1, 0x07030602u)};
-}
 
 // W6: one 16-code group's int8-grid values (decode_group<6>'s arithmetic: clamp(rint((code - 32) * s), +-127), with
 // (code - 32) * s formed exactly as code * s - 32 s) as bytes in column order. lo / hi: the nibble words of codes
@@ -2177,21 +2147,18 @@ static int check_rows(const char* what, int64_t plane, int32_t K, const int64_t*
   return 0;
 }
 
-int d3_expert_groups_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse,
-                             int32_t* groups, int32_t* work, int64_t work_ints, int32_t mode, int32_t rotate,
-                             const void* x, int32_t T, int32_t K, void* planes, float* scales, void* stream) {
-  if (!groups || !work || (P > 0 && (!ids || !order || !inverse))) return fail("d3_expert_groups_prep_i8: null pointer");
-  if (P < 0 || E < 1 || E > GROUPS_MAX_E) return fail("d3_expert_groups_prep_i8: 1 <= E <= 1024, P >= 0");
-  if (T > 0 && (!x || !planes || !scales)) return fail("d3_expert_groups_prep_i8: null pointer");
+static int groups_prep(const char* what, const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse,
+                       int32_t* groups, int32_t* work, int cap, int32_t* wide, int wide_cap, int32_t mode,
+                       int32_t rotate, const void* x, int32_t T, int32_t K, void* planes, float* scales,
+                       void* stream) {
+  if (P > 0 && (!ids || !order || !inverse)) return fail(std::string(what) + ": null pointer");
+  if (T > 0 && (!x || !planes || !scales)) return fail(std::string(what) + ": null pointer");
   if (T < 0 || (mode != 0 && mode != 1) || !supported_k(K))
-    return fail("d3_expert_groups_prep_i8: T >= 0, mode 0 (float32 rows) or 1 (bf16 rows), K in {256..2048}");
-  const int64_t need = d3_grouped_mfma_work_ints(E, P);
-  if (work_ints < need) return fail("d3_expert_groups_prep_i8: work holds fewer than d3_grouped_mfma_work_ints ints");
-  const int cap = (int)((need - 2) / 2);
+    return fail(std::string(what) + ": T >= 0, mode 0 (float32 rows) or 1 (bf16 rows), K in {256..2048}");
   const hipStream_t s = (hipStream_t)stream;
   const dim3 grid(1 + (T + 3) / 4);
   int8_t* pl = (int8_t*)planes;
-#define D3_GP(M, R) hipLaunchKernelGGL((groups_prep_kernel<M, R>), grid, dim3(1024), 0, s, ids, P, E, order, inverse, groups, work, cap, x, T, K, pl, scales)
+#define D3_GP(M, R) hipLaunchKernelGGL((groups_prep_kernel<M, R>), grid, dim3(1024), 0, s, ids, P, E, order, inverse, groups, work, cap, wide, wide_cap, x, T, K, pl, scales)
   switch (mode * 2 + (rotate ? 1 : 0)) {
     case 0: D3_GP(0, false); break;
     case 1: D3_GP(0, true); break;
@@ -2199,7 +2166,29 @@ int d3_expert_groups_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* 
     default: D3_GP(1, true); break;
   }
 #undef D3_GP
-  return done("d3_expert_groups_prep_i8");
+  return done(what);
+}
+
+int d3_expert_groups_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse,
+                             int32_t* groups, int32_t* work, int64_t work_ints, int32_t mode, int32_t rotate,
+                             const void* x, int32_t T, int32_t K, void* planes, float* scales, void* stream) {
+  if (!groups || !work) return fail("d3_expert_groups_prep_i8: null pointer");
+  if (P < 0 || E < 1 || E > GROUPS_MAX_E) return fail("d3_expert_groups_prep_i8: 1 <= E <= 1024, P >= 0");
+  const int64_t need = d3_grouped_mfma_work_ints(E, P);
+  if (work_ints < need) return fail("d3_expert_groups_prep_i8: work holds fewer than d3_grouped_mfma_work_ints ints");
+  return groups_prep("d3_expert_groups_prep_i8", ids, P, E, order, inverse, groups, work, (int)((need - 2) / 2),
+                     nullptr, 0, mode, rotate, x, T, K, planes, scales, stream);
+}
+
+int d3_prompt_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse, int32_t* passes,
+                      int64_t pass_ints, int32_t mode, int32_t rotate, const void* x, int32_t T, int32_t K,
+                      void* planes, float* scales, void* stream) {
+  if (!passes) return fail("d3_prompt_prep_i8: null pointer");
+  if (P < 0 || E < 1 || E > GROUPS_MAX_E) return fail("d3_prompt_prep_i8: 1 <= E <= 1024, P >= 0");
+  const int64_t need = d3_prompt_pass_ints(E, P);
+  if (pass_ints < need) return fail("d3_prompt_prep_i8: passes holds fewer than d3_prompt_pass_ints ints");
+  return groups_prep("d3_prompt_prep_i8", ids, P, E, order, inverse, nullptr, nullptr, 0, passes, (int)((need - 4) / 4),
+                     mode, rotate, x, T, K, planes, scales, stream);
 }
 
 int d3_grouped_fp8(const void* planes, int32_t n_planes, int64_t plane, const int64_t* order, int32_t k,

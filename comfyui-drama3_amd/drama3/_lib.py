@@ -91,6 +91,12 @@ SIGNATURES = {
     "d3_grouped_i8": (c_int32, [c_int32, c_void_p, c_void_p, c_int64, c_void_p, c_int32, c_int32, c_void_p, c_int32,
                                 c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                 c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p]),
+    "d3_prompt_pass_ints": (c_int64, [c_int32, c_int64]),
+    "d3_prompt_prep_i8": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_int32,
+                                    c_int32, c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p]),
+    "d3_prompt_i8": (c_int32, [c_int32, c_void_p, c_void_p, c_int64, c_void_p, c_int32, c_int32, c_void_p, c_int64,
+                               c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32,
+                               c_void_p]),
     "d3_combine_rows": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p,
                                   c_int32, c_void_p]),
     "d3_decode_codes": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p]),

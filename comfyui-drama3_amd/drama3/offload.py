@@ -383,6 +383,15 @@ def resident_prefill(x, topk_idx, topk_weight, banks, rows, kind, codebooks, num
     the pairs grouped by expert on the device, each product weighted and summed over k; x's dtype."""
     top_k = topk_idx.shape[1]
     planes = None
+    if topk_idx.is_cuda and kernels.prompt_wide_fits(kind, banks, rows, topk_idx.numel(), num_experts, x.shape[1]):
+        order, inverse, passes, planes, scales = kernels.prompt_prep_i8(topk_idx, num_experts, x, True)
+        P = order.shape[0]
+        hidden = kernels.prompt_i8(kind, planes, scales, P, x.shape[1], passes, num_experts, banks[0], codebooks[0],
+                                   rows[0], order, top_k, swiglu=True)
+        planes, scales = kernels.prep_planes_i8(hidden, True)
+        sorted_out = kernels.prompt_i8(kind, planes, scales, P, rows[0] // 2, passes, num_experts, banks[1],
+                                       codebooks[1], rows[1])
+        return _combine(sorted_out, inverse, topk_weight, x.dtype)
     if topk_idx.is_cuda and kind != "fp8" and rows[0] % 64 == 0 and rows[1] % 64 == 0:
         # one launch: the grouping, its plan of the grouped products' passes, and x's rows as int8 planes
         order, inverse, groups, work, *planes = kernels.expert_groups_prep_i8(topk_idx, num_experts, x, True)

@@ -294,6 +294,22 @@ int d3_grouped_i8(int32_t kind, const void* planes, const float* scales, int64_t
                   const void* host_w, const void* host_s, const void* host_c, const float* codebook, float* out,
                   int32_t N, int32_t K, void* stream);
 
+/* The same products for a long prompt on banks held whole on the GPU (expert e's N rows at e * N; offload.py:138-149
+ * with no slot cache): passes of up to 96 rows against 256 weight rows per workgroup. d3_prompt_prep_i8 does what
+ * d3_expert_groups_prep_i8 does, with the passes as its plan: passes [4 + 4 n] int32 (>= d3_prompt_pass_ints(E, P)),
+ * passes[0] their number, then (expert, first row in order, rows, 0) each. d3_prompt_i8 runs one bank (w, s, c: the
+ * expert fields, as host_w, host_s, host_c of d3_grouped_i8) over them, out [rows, N] float32 =
+ * scale * (S * (A0 + (A1 + A2 / 254) / 254)) as d3_grouped_i8, each step of the sum over the planes rounded once.
+ * With swiglu the bank's rows are N / 2 gate rows, then N / 2 up rows, and out [rows, N / 2] = SiLU(gate) * up.
+ * N % 256 == 0, K % 256 == 0 up to 2048, planes and w at 16-byte alignment, plane < 2^32 bytes. */
+int64_t d3_prompt_pass_ints(int32_t E, int64_t P);
+int d3_prompt_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse, int32_t* passes,
+                      int64_t pass_ints, int32_t mode, int32_t rotate, const void* x, int32_t T, int32_t K,
+                      void* planes, float* scales, void* stream);
+int d3_prompt_i8(int32_t kind, const void* planes, const float* scales, int64_t plane, const int64_t* order, int32_t k,
+                 int32_t rows, const int32_t* passes, int64_t pass_ints, int32_t E, const void* w, const void* s,
+                 const float* c, const float* codebook, float* out, int32_t N, int32_t K, int32_t swiglu, void* stream);
+
 /* The weighted sum over k (offload.py:144-149): out [T, H] = sum over j in order of weights[t, j] *
  * sorted_out[inverse[t k + j]] in float32 (pairs with inverse -1 left out), stored as float32 / bf16 / fp16
  * (out_type 0 / 1 / 2); weights [T, k] bf16 (weights_bf16) or float32. H % 4 == 0. */

@@ -1,0 +1,100 @@
+"""The wide products of a resident prompt (kernels.prompt_prep_i8 / prompt_i8) at the edges of their tiles, against the
+32-row products (grouped_i8, themselves pinned on the oracle) on the same planes, and their decoding against the
+oracle's. resident_prefill's own oracle tests with many rows per expert run through them too."""
+import numpy as np
+import pytest
+import torch
+
+from drama3 import kernels, offload
+from oracle import numerics
+from oracle import reference as ref
+from tests.test_gpu_ref import DEV, _bank, dev, fields_on, zipf_topk
+
+pytestmark = pytest.mark.gpu
+
+# rows per expert: none, one, around one 16-row tile, around a pass's 96 rows, two and three passes, an odd middle
+COUNTS = [0, 1, 15, 16, 17, 95, 96, 97, 193, 240, 50]
+
+
+@pytest.mark.parametrize("K, N", [(256, 512), (2048, 256), (768, 1024)])
+@pytest.mark.parametrize("kind", ["int8", "w4", "w6"])
+def test_prompt_products_match_the_32_row_products(kind, K, N):
+    """Both read the same int8 planes and add the same exact int32 sums A0, A1, A2 in float32, A0 + (A1 + A2 / 254) /
+    254, with the roundings of two divisions or of two fused steps: they differ by at most one rounding of the result
+    and two of (A1 + A2 / 254) / 254, which is under a hundredth of the row's largest result on these inputs, so by
+    less than 2^-22 of that. SwiGLU: SiLU(gate) * up of the same numbers, with a float32 exp and divide (2^-20)."""
+    rng = np.random.default_rng(len(kind) + K)
+    E, T = len(COUNTS), sum(COUNTS)
+    fields = fields_on(_bank(kind, rng, E, N, K))
+    cb = dev(ref.default_codebook()) if kind == "w4" else None
+    idx = dev(rng.permutation(np.repeat(np.arange(E), COUNTS)).astype(np.int64)).view(T, 1)
+    x = dev(rng.standard_normal((T, K)).astype(np.float32)).to(torch.bfloat16)
+    order, inverse, passes, planes, scales = kernels.prompt_prep_i8(idx, E, x, True)
+    listed = passes[4:4 + 4 * int(passes[0])].view(-1, 4).cpu().numpy()
+    assert listed[:, 2].sum() == T and listed[:, 2].min() >= 1 and listed[:, 2].max() <= 96
+    order2, inverse2, groups, work, planes2, scales2 = kernels.expert_groups_prep_i8(idx, E, x, True)
+    assert torch.equal(planes, planes2) and torch.equal(scales, scales2)
+    got = kernels.prompt_i8(kind, planes, scales, T, K, passes, E, fields, cb, N, order, 1)
+    want = kernels.grouped_i8(kind, planes, scales, T, K, groups, work, fields, fields, cb, N, order=order2, k=1)
+    got, want = got[inverse.long()].double(), want[inverse2.long()].double()  # by token
+    assert torch.all((got - want).abs() <= 2.0 ** -22 * want.abs().amax(dim=1, keepdim=True))
+    hidden = kernels.prompt_i8(kind, planes, scales, T, K, passes, E, fields, cb, N, order, 1, swiglu=True)
+    gate, up = got[:, :N // 2], got[:, N // 2:]
+    want = gate / (1 + torch.exp(-gate)) * up
+    assert torch.all((hidden[inverse.long()].double() - want).abs() <= 2.0 ** -20 * (want.abs() + gate.abs() * 1e-6))
+
+
+@pytest.mark.parametrize("kind", ["w4", "w6"])
+def test_prompt_products_decode_exactly(kind):
+    """One-hot rows make each output one decoded weight times its channel scale, a single product: bit for bit the
+    oracle's, for every scale byte but NaN's."""
+    rng = np.random.default_rng(len(kind))
+    E, N, K = 2, 256, 256
+    host = _bank(kind, rng, E, N, K)
+    finite = np.array([b for b in range(256) if b & 0x7F != 0x7F], np.uint8)
+    host["scale"] = rng.choice(finite, size=host["scale"].shape)
+    cb = ref.default_codebook()
+    fields = fields_on(host)
+    idx = dev(np.repeat(np.arange(E), K).astype(np.int64)).view(-1, 1)
+    x = torch.eye(K, device=DEV).repeat(E, 1)
+    order, inverse, passes, planes, scales = kernels.prompt_prep_i8(idx, E, x, False)
+    out = kernels.prompt_i8(kind, planes, scales, E * K, K, passes, E, fields, dev(cb) if kind == "w4" else None, N,
+                            order, 1)[inverse.long()].cpu().numpy()
+    w = ref.decode_codes_ref(host["_qdata"], host["scale"], int(kind[1]), cb).astype(np.float32)
+    w = w * host["s_channel"].reshape(-1, 1).astype(np.float32)
+    for e in range(E):
+        assert np.array_equal(out[e * K:(e + 1) * K], w[e * N:(e + 1) * N].T)
+
+
+@pytest.mark.parametrize("kind", ["int8", "w4", "w6"])
+def test_prompt_path_equals_the_32_row_path_and_replays(kind, monkeypatch):
+    """resident_prefill through the wide products and through the 32-row ones: bf16 results of float32 sums that differ
+    in their last bits, so within one bf16 step; captured in a graph, every replay equals the eager result bit for
+    bit, with other work in between."""
+    rng = np.random.default_rng(30 + len(kind))
+    E, T, k, H, I = 12, 333, 4, 2048, 512
+    banks = [fields_on(b) for b in (_bank(kind, rng, E, 2 * I, H), _bank(kind, rng, E, H, I))]
+    cb = dev(ref.default_codebook()) if kind == "w4" else None
+    idx = dev(zipf_topk(rng, T, E, k).astype(np.int64))
+    w = dev(numerics.bf16_round(rng.dirichlet(np.ones(k), T).astype(np.float32))).to(torch.bfloat16)
+    x = dev(rng.standard_normal((T, H)).astype(np.float32)).to(torch.bfloat16)
+    run = lambda: offload.resident_prefill(x, idx, w, banks, (2 * I, H), kind, (cb, cb), E)  # noqa: E731
+    assert kernels.prompt_wide_fits(kind, banks, (2 * I, H), T * k, E, H)
+    wide = run()
+    monkeypatch.setattr(kernels, "PROMPT_WIDE_ROWS", 10 ** 9)
+    narrow = run()
+    monkeypatch.undo()
+    a, b = wide.double(), narrow.double()
+    assert torch.all((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-5 * b.abs().max())
+    stream = torch.cuda.Stream(DEV)
+    stream.wait_stream(torch.cuda.current_stream(DEV))
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(g, stream=stream):
+            out = run()
+    torch.cuda.current_stream(DEV).wait_stream(stream)
+    for _ in range(3):
+        x.copy_(torch.randn(x.shape, device=DEV).to(torch.bfloat16))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), run().view(torch.int16))
