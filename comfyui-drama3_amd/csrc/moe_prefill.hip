@@ -17,8 +17,11 @@
 //   down       grid (H / 32, E): 32 output rows of one expert against its pairs; the product, scaled by the pair's
 //              routing weight, lands in the pair's own row
 //   reduce     out[t] = bf16(sum over the row's k pairs, in routing order)
+// With many pairs per expert the two products run as 256 x 256 tiles instead (a8_wide.hip; the grouping then plans
+// their passes).
 // Results do not depend on the order of pairs within an expert (every output element is its own dot product), so the
 // grouping may use atomics.
+#include "a8_wide.hpp"
 #include "formats.hpp"
 #include "../../include/drama3_moe.h"
 
@@ -74,8 +77,10 @@ D3_INLINE int wave_exclusive_scan(int v, int lane, int& total) {
 
 // (a workgroup of 1024 threads; ids may be in LDS or device memory; inv_lds, if given, gets each pair's sorted
 // position)
+// (wide > 0: the units of the wide products instead, passes of at most `wide` 16-row tiles, all of an expert's with the
+// same number but the last)
 D3_INLINE void group_pairs(const int64_t* ids, int P, int E, int* counts, int* offsets, int* perm, int4* units,
-                           int* meta, int* inv_lds = nullptr) {
+                           int* meta, int* inv_lds = nullptr, int wide = 0) {
   __shared__ int cnt[MAX_EXPERTS], cur[MAX_EXPERTS], by_rank[MAX_EXPERTS], rank_base[MAX_EXPERTS];
   __shared__ int used;
   const int tid = threadIdx.x;
@@ -120,23 +125,24 @@ D3_INLINE void group_pairs(const int64_t* ids, int P, int E, int* counts, int* o
   }
   __syncthreads();
   const int U = used;
+  auto unit_count = [&](int c) { return wide ? wt_passes(c, wide) : (c + UNIT_PAIRS - 1) / UNIT_PAIRS; };
   if (tid < 64) {
     const int per = (U + 63) / 64, lo = tid * per, hi = min(U, lo + per);
     int run = 0;
-    for (int r = lo; r < hi; r++) run += (cnt[by_rank[r]] + UNIT_PAIRS - 1) / UNIT_PAIRS;
+    for (int r = lo; r < hi; r++) run += unit_count(cnt[by_rank[r]]);
     int total;
     int at = wave_exclusive_scan(run, tid, total);
     for (int r = lo; r < hi; r++) {
       rank_base[r] = at;
-      at += (cnt[by_rank[r]] + UNIT_PAIRS - 1) / UNIT_PAIRS;
+      at += unit_count(cnt[by_rank[r]]);
     }
     if (tid == 0) meta[0] = total;
   }
   __syncthreads();
   for (int r = tid; r < U; r += 1024) {
     const int e = by_rank[r], c = cnt[e], first = cur[e];
-    for (int u = 0; u * UNIT_PAIRS < c; u++)
-      units[rank_base[r] + u] = int4{e, first + u * UNIT_PAIRS, min(UNIT_PAIRS, c - u * UNIT_PAIRS), 0};
+    const int step = wide ? 16 * wt_tiles(c, wide) : UNIT_PAIRS;
+    for (int u = 0; u * step < c; u++) units[rank_base[r] + u] = int4{e, first + u * step, min(step, c - u * step), 0};
   }
   __syncthreads();
   for (int p = tid; p < P; p += 1024) {
@@ -147,8 +153,8 @@ D3_INLINE void group_pairs(const int64_t* ids, int P, int E, int* counts, int* o
 }
 
 __global__ void __launch_bounds__(1024) group_kernel(const int64_t* ids, int P, int E, int* counts, int* offsets,
-                                                     int* perm, int4* units, int* meta) {
-  group_pairs(ids, P, E, counts, offsets, perm, units, meta);
+                                                     int* perm, int4* units, int* meta, int wide) {
+  group_pairs(ids, P, E, counts, offsets, perm, units, meta, nullptr, wide);
 }
 
 // One row of x (bf16, H columns; lane l holds columns 512 c + 8 l .. + 7 in xr[c]) quantized per row: codes in the
@@ -400,13 +406,13 @@ D3_INLINE void load_weights(Weights<F, Geometry<F, H, I, MODE>::SW>& wt, const P
 // epilogue and barriers: 164.6 / 164.3 us against 167.8 / 167.7. (Group-scaled weights kept two workgroups per CU
 // that way: W4A8 128.2 against 125.8.) Activation rows are read without a branch (columns past the unit's pairs
 // read its first pair and their products are never stored). colv / colp: per column (pair) of a tile, its epilogue
-// scale and (down) its pair index, staged in LDS by wave 0.
+// scale and (down) its pair index, staged in LDS by wave 0; rowv (int8): the item's row scales.
 constexpr bool late_weights(int F) { return !group_scaled(F); }
 template <int F, int H, int I, int MODE>
 D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
                             const Weights<F, Geometry<F, H, I, MODE>::SW>& wt, int4 unit_n, int4 unit, int it,
                             int c0, const float* gs, float (*part)[Geometry<F, H, I, MODE>::KS][16][17], float* colv,
-                            int* colp, int& pr, Weights<F, Geometry<F, H, I, MODE>::SW>* next_wt, int it_n) {
+                            int* colp, float* rowv, int& pr, Weights<F, Geometry<F, H, I, MODE>::SW>* next_wt, int it_n) {
   using G = Geometry<F, H, I, MODE>;
   constexpr int SW = G::SW, KS = G::KS, K = G::K, STEPS = K / 128;
   constexpr int SHIFT = unpack_shift(F);
@@ -451,11 +457,15 @@ D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
 #pragma unroll
       for (int i = 0; i < 4; i++) y[i] = acc[i] * wt.rs[t][i];
     } else if constexpr (F == FMT_I8) {
+      // the slices' int32 sums meet exactly; the row scale comes after (in LDS, as its bits)
       i32x4 acc = {0, 0, 0, 0};
 #pragma unroll
       for (int j = 0; j < SW; j++) acc = step_i8<F>(wt.raw[t][j], lo[j], hi[j], acc);
+      y = __builtin_bit_cast(f32x4, acc);
+      if (ks == 0 && c0 == 0 && col == 0) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) y[i] = (float)acc[i] * wt.rs[t][i];
+        for (int i = 0; i < 4; i++) rowv[16 * (2 * tp + t) + 4 * q + i] = wt.rs[t][i];
+      }
     } else {
       const float* g = gs + (2 * tp + t) * 16 * STEPS;
       f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -477,10 +487,21 @@ D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
     const int u = tid & 15, j = tid >> 4;
     if (c0 + j < n) {
       float gv = 0.0f, uv = 0.0f;
+      if constexpr (F == FMT_I8) {
+        int g = 0, up = 0;
 #pragma unroll
-      for (int k2 = 0; k2 < KS; k2++) {
-        gv += part[0][k2][u][j];
-        uv += part[1][k2][u][j];
+        for (int k2 = 0; k2 < KS; k2++) {
+          g += __float_as_int(part[0][k2][u][j]);
+          up += __float_as_int(part[1][k2][u][j]);
+        }
+        gv = (float)g * rowv[u];
+        uv = (float)up * rowv[16 + u];
+      } else {
+#pragma unroll
+        for (int k2 = 0; k2 < KS; k2++) {
+          gv += part[0][k2][u][j];
+          uv += part[1][k2][u][j];
+        }
       }
       const float xs = colv[j];
       gv *= xs;
@@ -494,8 +515,15 @@ D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
       const int o = tid + 256 * r4, r = o & 63, j = o >> 6;
       if (c0 + j < n) {
         float v = 0.0f;
+        if constexpr (F == FMT_I8) {
+          int d = 0;
 #pragma unroll
-        for (int k2 = 0; k2 < KS; k2++) v += part[r >> 4][k2][r & 15][j];
+          for (int k2 = 0; k2 < KS; k2++) d += __float_as_int(part[r >> 4][k2][r & 15][j]);
+          v = (float)d * rowv[r];
+        } else {
+#pragma unroll
+          for (int k2 = 0; k2 < KS; k2++) v += part[r >> 4][k2][r & 15][j];
+        }
         a.parts[(size_t)colp[j] * H + 64 * it + r] = v * colv[j];
       }
     }
@@ -508,7 +536,7 @@ template <int F, int H, int I, int MODE>
 D3_INLINE void compute_item(const PrefillArgs& a, const int* __restrict__ perm,
                             Weights<F, Geometry<F, H, I, MODE>::SW>& wt, int4 unit_n, int4 unit, int it,
                             float* gs, float (*part)[Geometry<F, H, I, MODE>::KS][16][17], float* colv, int* colp,
-                            int& pr, bool more, int it_n) {
+                            float* rowv, int& pr, bool more, int it_n) {
   using G = Geometry<F, H, I, MODE>;
   constexpr int STEPS = G::K / 128;
   const int tid = threadIdx.x;
@@ -524,12 +552,12 @@ D3_INLINE void compute_item(const PrefillArgs& a, const int* __restrict__ perm,
   const int last = (unit.z - 1) & ~15;
   if constexpr (late_weights(F)) {
     for (int c0 = 0; c0 < last; c0 += 16)
-      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, pr, nullptr, 0);
-    compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, last, gs, part, colv, colp, pr, more ? &wt : nullptr,
+      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, rowv, pr, nullptr, 0);
+    compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, last, gs, part, colv, colp, rowv, pr, more ? &wt : nullptr,
                                 it_n);
   } else {
     for (int c0 = 0; c0 <= last; c0 += 16)
-      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, pr, nullptr, 0);
+      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, rowv, pr, nullptr, 0);
   }
 }
 
@@ -543,6 +571,7 @@ __global__ void __launch_bounds__(256) grouped_kernel(PrefillArgs a, const int4*
   __shared__ float gs[group_scaled(F) ? G::TILES * 16 * (G::K / 128) : 1];
   __shared__ float colv[16];
   __shared__ int colp[16];
+  __shared__ float rowv[F == FMT_I8 ? G::TILES * 16 : 1];
   const int n_items = meta[0] * G::PER_EXPERT;
   int i = blockIdx.x;
   if (i >= n_items) return;
@@ -563,7 +592,7 @@ __global__ void __launch_bounds__(256) grouped_kernel(PrefillArgs a, const int4*
     const bool more = in < n_items;
     const int4 unit_n = units[(more ? in : i) / G::PER_EXPERT];
     const int it_n = (more ? in : i) % G::PER_EXPERT;
-    compute_item<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, gs, part, colv, colp, pr, more, it_n);
+    compute_item<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, gs, part, colv, colp, rowv, pr, more, it_n);
     if (!more) break;
     i = in;
     rnd++;
@@ -659,9 +688,49 @@ template <int F, int WIDTH> void launch_quantize(const float* src, int rows, uin
                      pair_weight, perm);
 }
 
+// From this many pairs per expert on average, the wide products (a8_wide.hip) in place of the grouped ones. Below, a
+// pass has too few rows to pay for its 256-row tile, and one workgroup per CU keeps fewer bytes on their way. Measured,
+// us per layer (grouped / wide), 128 experts with FFN 768 and 256 with FFN 512, even routing: int8 at 32 pairs 190 / 167
+// and 258 / 237 (Zipf(1.1) 195 / 200 and 277 / 257; at 37.5 218 / 207); W4 at 52 212 / 173 and 292 / 253 (Zipf 225 /
+// 217, 308 / 288; at 44 198 / 212); W6 at 52 243 / 212 and 342 / 316 (Zipf 262 / 260, 375 / 353; at 44 232 / 256): the
+// codes are read at half or three quarters the bytes, so their grouped products hold out longer.
+constexpr int A8_WIDE_PAIRS = 34, A8_WIDE_PAIRS_CODES = 52;
+// (16-byte aligned banks: the copies to LDS need it; row offsets in 32 bits)
+bool wide_fits(const d3_moe_a8_prefill_desc& d) {
+  const int64_t P = (int64_t)d.T * d.topk;
+  return P >= (int64_t)(group_scaled(d.format) ? A8_WIDE_PAIRS_CODES : A8_WIDE_PAIRS) * d.E && (((uintptr_t)d.gate_up | (uintptr_t)d.down) & 15) == 0 &&
+         std::max((int64_t)d.T * d.H, P * d.I) < ((int64_t)1 << 32) - 4096;
+}
+
 template <int F, int H, int I> void run(const PrefillArgs& pa, const d3_moe_a8_prefill_desc& d, const Layout& L,
                                         uint8_t* ws, hipStream_t s) {
   const int P = d.T * d.topk;
+  if (wide_fits(d)) {
+    A8WideArgs a;
+    a.perm = pa.perm;
+    a.k = d.topk;
+    a.count = pa.meta;
+    a.passes = pa.units;
+    const int cap = std::min(d.E, P) + P / (16 * a8_wide_tiles(F));
+    a.act = pa.xq;
+    a.act_scale = pa.xs;
+    a.w = pa.gu_w;
+    a.s = pa.gu_s;
+    a.out = pa.h;
+    a.N = 2 * I;
+    a.K = H;
+    launch_a8_wide(F, false, a, cap, s);
+    launch_quantize<F, I>((const float*)(ws + L.h), P, ws + L.hq, (float*)(ws + L.hs), pa.weights, pa.perm, s);
+    a.act = pa.hq;
+    a.act_scale = pa.hs;
+    a.w = pa.dn_w;
+    a.s = pa.dn_s;
+    a.out = pa.parts;
+    a.N = H;
+    a.K = I;
+    launch_a8_wide(F, true, a, cap, s);
+    return;
+  }
   const int max_units = std::min(d.E, P) + P / UNIT_PAIRS;
   launch_products<F, H, I>(pa, max_units, s);
   launch_quantize<F, I>((const float*)(ws + L.h), P, ws + L.hq, (float*)(ws + L.hs), pa.weights, pa.perm, s);
@@ -699,7 +768,7 @@ int d3_moe_a8_prefill(const d3_moe_a8_prefill_desc* d, void* stream) {
   // up to 16 rows: routing, x's quantization and the grouping in one launch (one workgroup). Measured on a 2048 x
   // 768, 128-expert layer, us per layer against the wide launches (then route, group and quantize): int8 66.6 / 70.8 at 7 rows, 70.2 / 74.0 at 8, 84.2 / 87.1 at 12, 97.2 / 98.6 at 16; W4A8
   // 52.1 / 56.6, 55.5 / 59.8, 64.3 / 67.3, 73.6 / 75.3.
-  const bool small = d->T <= 16 && d->topk <= 8 && d->E <= 256;
+  const bool small = d->T <= 16 && d->topk <= 8 && d->E <= 256 && !wide_fits(*d);
   if (small) {
     SmallPrepArgs sa;
     sa.logits = (const uint16_t*)d->logits;
@@ -740,7 +809,8 @@ int d3_moe_a8_prefill(const d3_moe_a8_prefill_desc* d, void* stream) {
   }
   if (!small)
     hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), 0, s, (const int64_t*)ids, P, d->E, (int*)(ws + L.counts),
-                       (int*)(ws + L.offsets), (int*)(ws + L.perm), (int4*)(ws + L.units), (int*)(ws + L.meta));
+                       (int*)(ws + L.offsets), (int*)(ws + L.perm), (int4*)(ws + L.units), (int*)(ws + L.meta),
+                       wide_fits(*d) ? a8_wide_tiles(d->format) : 0);
   PrefillArgs pa;
   pa.ids = ids;
   pa.weights = weights;

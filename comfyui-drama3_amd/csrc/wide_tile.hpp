@@ -22,7 +22,14 @@ D3_INLINE uint32_t lds_address(const void* p) {
 // passing through registers. The compiler does not count these loads: dma_wait() before the barrier that hands them to
 // the other waves.
 D3_INLINE void dma16(uint32_t lds, const void* base, uint32_t off) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(off), "s"(base) : "memory");
+  // (both uniform already; said again for the compiler, which may keep a loop's pointers in vector registers)
+  const uint64_t at = (uint64_t)base;
+  const uint64_t sbase = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at) |
+                         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32;
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(off), "s"(sbase)
+               : "memory");
 }
 D3_INLINE void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

@@ -245,3 +245,38 @@ def test_prefill_rows_independent_at_1024_rows(fmt):
     for r in (0, int(hot_rows[0])):
         one = moe.moe_prefill(x[r:r + 1], gate_up, down, 8, logits=logits[r:r + 1])
         assert torch.equal(one, out[r:r + 1])
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_prefill_wide_products_match_oracle(fmt):
+    """Enough pairs per expert (54 on average) for the wide products: against the oracle at the layer bars."""
+    gate_up, down = banks(fmt)
+    gen = torch.Generator(device=DEV).manual_seed(60 + fmt)
+    x = torch.randn((108, H), generator=gen, device=DEV).to(torch.bfloat16)
+    logits = torch.randn((108, 16), generator=gen, device=DEV).to(torch.bfloat16)
+    check(fmt, x, logits, gate_up, down)
+
+
+@pytest.mark.parametrize("inter", [768, 512])
+@pytest.mark.parametrize("fmt", FMTS)
+def test_prefill_wide_products_at_tile_edges(fmt, inter):
+    """Experts with 0, 1, 15 .. 17, 255 .. 257, 300 and 530 rows, one and two per token: a row's output depends on that
+    row alone, so the wide products' rows equal the same rows run a few at a time (the grouped products, pinned on the
+    oracle) at the layer bars: their float32 sums differ in order, which can move a hidden code by one step."""
+    gate_up, down = banks(fmt, inter=inter)
+    counts = [0, 1, 15, 16, 17, 31, 33, 95, 0, 255, 256, 257, 300, 530, 2, 64]
+    rng = np.random.default_rng(fmt)
+    ids = rng.permutation(np.repeat(np.arange(16), counts))
+    T = len(ids)
+    idx = torch.from_numpy(np.stack([ids, (ids + 1 + rng.integers(0, 15, T)) % 16], axis=1)).to(DEV)
+    gen = torch.Generator(device=DEV).manual_seed(61)
+    w = torch.rand((T, 2), generator=gen, device=DEV)
+    x = torch.randn((T, H), generator=gen, device=DEV).to(torch.bfloat16)
+    for k in (1, 2):
+        i, v = idx[:, :k].contiguous(), w[:, :k].contiguous()
+        got = moe.moe_prefill(x, gate_up, down, k, topk_idx=i, topk_weight=v).float().cpu().numpy()
+        part = [moe.moe_prefill(x[t:t + 200], gate_up, down, k, topk_idx=i[t:t + 200], topk_weight=v[t:t + 200])
+                for t in range(0, T, 200)]
+        want = torch.cat(part).float().cpu().numpy()
+        assert np.all(np.isfinite(got))
+        assert_layer_close(fmt, got.astype(np.float64), want.astype(np.float64))
