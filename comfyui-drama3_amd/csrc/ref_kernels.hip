@@ -665,8 +665,9 @@ D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* ord
 }
 
 __global__ void __launch_bounds__(1024) expert_groups_kernel(const int64_t* ids, int P, int E, int64_t* order,
-                                                             int* inverse, int* groups, int* work, int cap) {
-  expert_groups_body(ids, P, E, order, inverse, groups, work, cap, nullptr, 0);
+                                                             int* inverse, int* groups, int* work, int cap,
+                                                             int* wide, int wide_cap) {
+  expert_groups_body(ids, P, E, order, inverse, groups, work, cap, wide, wide_cap);
 }
 
 // columns c0 .. c0 + 3 of row `row` of x as float (SRC as for prep_planes_kernel)
@@ -2237,8 +2238,19 @@ int d3_expert_groups(const int64_t* ids, int32_t P, int32_t E, int64_t* order, i
     cap = (int)((need - 2) / 2);
   }
   hipLaunchKernelGGL(expert_groups_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, P, E, order, inverse,
-                     groups, work, cap);
+                     groups, work, cap, nullptr, 0);
   return done("d3_expert_groups");
+}
+
+int d3_prompt_groups(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse, int32_t* passes,
+                     int64_t pass_ints, void* stream) {
+  if (!passes || (P > 0 && (!ids || !order || !inverse))) return fail("d3_prompt_groups: null pointer");
+  if (P < 0 || E < 1 || E > GROUPS_MAX_E) return fail("d3_prompt_groups: 1 <= E <= 1024, P >= 0");
+  const int64_t need = d3_prompt_pass_ints(E, P);
+  if (pass_ints < need) return fail("d3_prompt_groups: passes holds fewer than d3_prompt_pass_ints ints");
+  hipLaunchKernelGGL(expert_groups_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, P, E, order, inverse,
+                     nullptr, nullptr, 0, passes, (int)((need - 4) / 4));
+  return done("d3_prompt_groups");
 }
 
 int d3_prep_planes(int32_t mode, int32_t rotate, int32_t n_planes, const void* x, const int64_t* order, int32_t k,

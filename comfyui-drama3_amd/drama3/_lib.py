@@ -97,6 +97,9 @@ SIGNATURES = {
     "d3_prompt_i8": (c_int32, [c_int32, c_void_p, c_void_p, c_int64, c_void_p, c_int32, c_int32, c_void_p, c_int64,
                                c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32,
                                c_void_p]),
+    "d3_prompt_groups": (c_int32, [c_void_p, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    "d3_prompt_fp8": (c_int32, [c_void_p, c_int32, c_int64, c_void_p, c_int32, c_int32, c_void_p, c_int64, c_int32,
+                                c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_void_p]),
     "d3_combine_rows": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_void_p,
                                   c_int32, c_void_p]),
     "d3_decode_codes": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_void_p, c_void_p]),

@@ -291,25 +291,40 @@ def expert_groups_prep_i8(topk_idx, num_experts, x, rotate):
     return order, inverse, groups, work, planes, scales
 
 
-# From this many rows an expert on average (pairs / experts), a resident prompt's integer products run in wide passes
+# From this many rows an expert on average (pairs / experts), a resident prompt's products run in wide passes
 # (96 rows against 256 weight rows per workgroup, each weight read from L2 and decoded once per pass) instead of
-# grouped_i8's 32-row passes, which keep more weight bytes on their way while the experts have few rows. Measured us per
+# 32-row passes, which keep more weight bytes on their way while the experts have few rows. Measured us per
 # layer (32-row / wide), top-8 of 128 experts with FFN 768, Zipf(1.1) and even routing: int8 24 rows 192 / 199 and 164 /
 # 170, 32 rows 219 / 209 and 213 / 183; W4 24 rows 212 / 231 and 191 / 193, 32 rows 241 / 239 and 241 / 199; W6 24 rows
-# 308 / 312 and 256 / 261, 32 rows 342 / 319 and 330 / 267. 256 experts with FFN 512 cross between 20 and 28.
+# 308 / 312 and 256 / 261, 32 rows 342 / 319 and 330 / 267; fp8 24 rows 213 / 214 and 188 / 179, 32 rows 248 / 225 and
+# 230 / 193. 256 experts with FFN 512 cross between 20 and 28.
 PROMPT_WIDE_ROWS = 30
 
 
 def prompt_wide_fits(kind, banks, rows, pairs, num_experts, width):
-    """Whether a resident prompt of `pairs` (row, expert) pairs over rows of `width` columns runs on prompt_prep_i8 and
-    prompt_i8: an integer kind, bank sizes in whole tiles, 16-byte aligned banks, planes under 2^32 bytes, and enough
-    rows per expert."""
-    if kind not in ("int8", "w4", "w6") or pairs < PROMPT_WIDE_ROWS * num_experts or num_experts > 1024:
+    """Whether a resident prompt of `pairs` (row, expert) pairs over rows of `width` columns runs on prompt_i8 /
+    prompt_fp8: bank sizes in whole tiles, aligned banks, planes under 2^32 bytes, and enough rows per expert."""
+    if pairs < PROMPT_WIDE_ROWS * num_experts or num_experts > 1024:
         return False
     inner = rows[0] // 2
+    weight, size = ("weight", 2) if kind == "fp8" else ("_qdata", 1)
     return (rows[0] % 512 == 0 and rows[1] % 256 == 0 and width % 256 == 0 and max(width, inner) <= 2048
-            and pairs * max(width, inner) < 2 ** 32 - 4096
-            and all(bank["_qdata"].data_ptr() % 16 == 0 and bank["scale"].data_ptr() % 4 == 0 for bank in banks))
+            and pairs * max(width, inner) * size < 2 ** 32 - 4096
+            and all(bank[weight].data_ptr() % 16 == 0 and bank["scale"].data_ptr() % 4 == 0 for bank in banks))
+
+
+def prompt_groups(topk_idx, num_experts):
+    """(order, inverse, passes): expert_groups with the wide products' plan."""
+    ids = topk_idx.reshape(-1).contiguous()
+    if ids.dtype != torch.int64:
+        ids = ids.long()
+    P = ids.shape[0]
+    order = torch.empty(P, dtype=torch.int64, device=ids.device)
+    inverse = torch.empty(P, dtype=torch.int32, device=ids.device)
+    ints = _lib.lib().d3_prompt_pass_ints(num_experts, P)
+    passes = torch.empty(ints, dtype=torch.int32, device=ids.device)
+    _call("d3_prompt_groups", _p(ids), P, num_experts, _p(order), _p(inverse), _p(passes), ints, _stream(ids))
+    return order, inverse, passes
 
 
 def prompt_prep_i8(topk_idx, num_experts, x, rotate):
@@ -341,6 +356,15 @@ def prompt_i8(kind, planes, scales, rows, width, passes, num_experts, fields, co
     _call("d3_prompt_i8", code, _p(planes), _p(scales), planes.shape[1], _p(order), int(k), rows, _p(passes),
           passes.shape[0], num_experts, _p(fields[wkey]), _p(fields["scale"]), _p(fields.get("s_channel")),
           _p(codebook), _p(out), n, width, int(swiglu), _stream(planes))
+    return out
+
+
+def prompt_fp8(planes, rows, width, passes, num_experts, fields, n, order=None, k=1, swiglu=False):
+    """prompt_i8 for an FP8 bank, over bf16 planes [1 or 3, R * width] (as grouped_fp8_planes)."""
+    out = torch.empty((rows, n // 2 if swiglu else n), dtype=torch.float32, device=planes.device)
+    _call("d3_prompt_fp8", _p(planes), planes.shape[0], planes.shape[1], _p(order), int(k), rows, _p(passes),
+          passes.shape[0], num_experts, _p(fields["weight"]), _p(fields["scale"]), _p(out), n, width, int(swiglu),
+          _stream(planes))
     return out
 
 

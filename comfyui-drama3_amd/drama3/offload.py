@@ -378,19 +378,33 @@ def _combine(sorted_out, inverse, topk_weight, dtype):
     return pairs.view(num_tokens, top_k, -1).sum(dim=1).to(dtype)
 
 
+def _wide_pairs(x, topk_idx, banks, rows, kind, codebooks, num_experts):
+    """(the pairs' rows through their experts [T * k, H] float32, inverse): resident_prefill's products in wide passes,
+    SiLU(gate) * up formed with the first bank's."""
+    top_k, width, inner = topk_idx.shape[1], x.shape[1], rows[0] // 2
+    if kind == "fp8":
+        order, inverse, passes = kernels.prompt_groups(topk_idx, num_experts)
+        planes = x.contiguous().view(1, -1) if x.dtype == torch.bfloat16 else kernels.prep_planes(x, False)
+        P = order.shape[0]
+        hidden = kernels.prompt_fp8(planes, P, width, passes, num_experts, banks[0], rows[0], order, top_k, swiglu=True)
+        planes = kernels.prep_planes(hidden, False)
+        return kernels.prompt_fp8(planes, P, inner, passes, num_experts, banks[1], rows[1]), inverse
+    order, inverse, passes, planes, scales = kernels.prompt_prep_i8(topk_idx, num_experts, x, True)
+    P = order.shape[0]
+    hidden = kernels.prompt_i8(kind, planes, scales, P, width, passes, num_experts, banks[0], codebooks[0], rows[0],
+                               order, top_k, swiglu=True)
+    planes, scales = kernels.prep_planes_i8(hidden, True)
+    return kernels.prompt_i8(kind, planes, scales, P, inner, passes, num_experts, banks[1], codebooks[1],
+                             rows[1]), inverse
+
+
 def resident_prefill(x, topk_idx, topk_weight, banks, rows, kind, codebooks, num_experts):
     """Many rows x [T, H] through banks held whole on the GPU (offload.py:138-149): one grouped kernel per bank over
     the pairs grouped by expert on the device, each product weighted and summed over k; x's dtype."""
     top_k = topk_idx.shape[1]
     planes = None
     if topk_idx.is_cuda and kernels.prompt_wide_fits(kind, banks, rows, topk_idx.numel(), num_experts, x.shape[1]):
-        order, inverse, passes, planes, scales = kernels.prompt_prep_i8(topk_idx, num_experts, x, True)
-        P = order.shape[0]
-        hidden = kernels.prompt_i8(kind, planes, scales, P, x.shape[1], passes, num_experts, banks[0], codebooks[0],
-                                   rows[0], order, top_k, swiglu=True)
-        planes, scales = kernels.prep_planes_i8(hidden, True)
-        sorted_out = kernels.prompt_i8(kind, planes, scales, P, rows[0] // 2, passes, num_experts, banks[1],
-                                       codebooks[1], rows[1])
+        sorted_out, inverse = _wide_pairs(x, topk_idx, banks, rows, kind, codebooks, num_experts)
         return _combine(sorted_out, inverse, topk_weight, x.dtype)
     if topk_idx.is_cuda and kind != "fp8" and rows[0] % 64 == 0 and rows[1] % 64 == 0:
         # one launch: the grouping, its plan of the grouped products' passes, and x's rows as int8 planes

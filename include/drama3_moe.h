@@ -309,6 +309,13 @@ int d3_prompt_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* order, 
 int d3_prompt_i8(int32_t kind, const void* planes, const float* scales, int64_t plane, const int64_t* order, int32_t k,
                  int32_t rows, const int32_t* passes, int64_t pass_ints, int32_t E, const void* w, const void* s,
                  const float* c, const float* codebook, float* out, int32_t N, int32_t K, int32_t swiglu, void* stream);
+/* The fp8 counterparts: d3_prompt_groups is the grouping and its passes alone, d3_prompt_fp8 one bank (w [E * N, K]
+ * e4m3, s [E * N / 128, K / 128]) over them, rows as d3_grouped_fp8's bf16 planes; the other arguments as above. */
+int d3_prompt_groups(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse, int32_t* passes,
+                     int64_t pass_ints, void* stream);
+int d3_prompt_fp8(const void* planes, int32_t n_planes, int64_t plane, const int64_t* order, int32_t k, int32_t rows,
+                  const int32_t* passes, int64_t pass_ints, int32_t E, const void* w, const float* s, float* out,
+                  int32_t N, int32_t K, int32_t swiglu, void* stream);
 
 /* The weighted sum over k (offload.py:144-149): out [T, H] = sum over j in order of weights[t, j] *
  * sorted_out[inverse[t k + j]] in float32 (pairs with inverse -1 left out), stored as float32 / bf16 / fp16

@@ -1,4 +1,4 @@
-"""The wide products of a resident prompt (kernels.prompt_prep_i8 / prompt_i8) at the edges of their tiles, against the
+"""The wide products of a resident prompt (kernels.prompt_i8 and prompt_fp8) at the edges of their tiles, against the
 32-row products (grouped_i8, themselves pinned on the oracle) on the same planes, and their decoding against the
 oracle's. resident_prefill's own oracle tests with many rows per expert run through them too."""
 import numpy as np
@@ -66,7 +66,49 @@ def test_prompt_products_decode_exactly(kind):
         assert np.array_equal(out[e * K:(e + 1) * K], w[e * N:(e + 1) * N].T)
 
 
-@pytest.mark.parametrize("kind", ["int8", "w4", "w6"])
+@pytest.mark.parametrize("planes", [1, 3])
+@pytest.mark.parametrize("K, N", [(256, 512), (2048, 256), (768, 1024)])
+def test_prompt_fp8_products_match_the_32_row_products(K, N, planes):
+    """Over bf16 rows and over float32 rows as three planes: float32 sums of the same exact products in another order,
+    each within 3e-5 of the sum of |w x| (the bar of the grouped products against the oracle)."""
+    rng = np.random.default_rng(K + planes)
+    E, T = len(COUNTS), sum(COUNTS)
+    host = _bank("fp8", rng, E, N, K)
+    fields = fields_on(host)
+    idx = dev(rng.permutation(np.repeat(np.arange(E), COUNTS)).astype(np.int64)).view(T, 1)
+    x = dev(rng.standard_normal((T, K)).astype(np.float32))
+    x = x.to(torch.bfloat16) if planes == 1 else x
+    split = x.view(1, -1) if planes == 1 else kernels.prep_planes(x, False)
+    order, inverse, passes = kernels.prompt_groups(idx, E)
+    order2, inverse2, groups, work = kernels.expert_groups(idx, E, plan=True)
+    got = kernels.prompt_fp8(split, T, K, passes, E, fields, N, order, 1)[inverse.long()].double()
+    want = kernels.grouped_fp8_planes(split, T, K, groups, work, fields, fields, N, order=order2, k=1)
+    want = want[inverse2.long()].double()
+    absw = dev(np.abs(ref.fp8_rows(host["weight"], host["scale"]))).double().view(E, N, K)
+    for e in range(E):
+        t = idx[:, 0] == e
+        assert torch.all((got[t] - want[t]).abs() <= 3e-5 * (x[t].double().abs() @ absw[e].T))
+    hidden = kernels.prompt_fp8(split, T, K, passes, E, fields, N, order, 1, swiglu=True)[inverse.long()].double()
+    gate, up = got[:, :N // 2], got[:, N // 2:]
+    want = gate / (1 + torch.exp(-gate)) * up
+    assert torch.all((hidden - want).abs() <= 2.0 ** -20 * (want.abs() + gate.abs() * 1e-6))
+
+
+def test_prompt_fp8_products_decode_exactly():
+    """One-hot rows make each output one e4m3 code times its block scale, bit for bit the oracle's."""
+    rng = np.random.default_rng(8)
+    E, N, K = 2, 256, 256
+    host = _bank("fp8", rng, E, N, K)
+    idx = dev(np.repeat(np.arange(E), K).astype(np.int64)).view(-1, 1)
+    x = torch.eye(K, device=DEV, dtype=torch.bfloat16).repeat(E, 1)
+    order, inverse, passes = kernels.prompt_groups(idx, E)
+    out = kernels.prompt_fp8(x.view(1, -1), E * K, K, passes, E, fields_on(host), N, order, 1)[inverse.long()]
+    w = ref.fp8_rows(host["weight"], host["scale"]).astype(np.float32)
+    for e in range(E):
+        assert np.array_equal(out[e * K:(e + 1) * K].cpu().numpy(), w[e * N:(e + 1) * N].T)
+
+
+@pytest.mark.parametrize("kind", ["int8", "fp8", "w4", "w6"])
 def test_prompt_path_equals_the_32_row_path_and_replays(kind, monkeypatch):
     """resident_prefill through the wide products and through the 32-row ones: bf16 results of float32 sums that differ
     in their last bits, so within one bf16 step; captured in a graph, every replay equals the eager result bit for
