@@ -23,6 +23,7 @@
 // grouping may use atomics.
 #include "a8_wide.hpp"
 #include "formats.hpp"
+#include "prompt_group.hpp"
 #include "../../include/drama3_moe.h"
 
 #include <algorithm>
@@ -77,10 +78,8 @@ D3_INLINE int wave_exclusive_scan(int v, int lane, int& total) {
 
 // (a workgroup of 1024 threads; ids may be in LDS or device memory; inv_lds, if given, gets each pair's sorted
 // position)
-// (wide > 0: the units of the wide products instead, passes of at most `wide` 16-row tiles, all of an expert's with the
-// same number but the last)
 D3_INLINE void group_pairs(const int64_t* ids, int P, int E, int* counts, int* offsets, int* perm, int4* units,
-                           int* meta, int* inv_lds = nullptr, int wide = 0) {
+                           int* meta, int* inv_lds = nullptr) {
   __shared__ int cnt[MAX_EXPERTS], cur[MAX_EXPERTS], by_rank[MAX_EXPERTS], rank_base[MAX_EXPERTS];
   __shared__ int used;
   const int tid = threadIdx.x;
@@ -125,24 +124,23 @@ D3_INLINE void group_pairs(const int64_t* ids, int P, int E, int* counts, int* o
   }
   __syncthreads();
   const int U = used;
-  auto unit_count = [&](int c) { return wide ? wt_passes(c, wide) : (c + UNIT_PAIRS - 1) / UNIT_PAIRS; };
   if (tid < 64) {
     const int per = (U + 63) / 64, lo = tid * per, hi = min(U, lo + per);
     int run = 0;
-    for (int r = lo; r < hi; r++) run += unit_count(cnt[by_rank[r]]);
+    for (int r = lo; r < hi; r++) run += (cnt[by_rank[r]] + UNIT_PAIRS - 1) / UNIT_PAIRS;
     int total;
     int at = wave_exclusive_scan(run, tid, total);
     for (int r = lo; r < hi; r++) {
       rank_base[r] = at;
-      at += unit_count(cnt[by_rank[r]]);
+      at += (cnt[by_rank[r]] + UNIT_PAIRS - 1) / UNIT_PAIRS;
     }
     if (tid == 0) meta[0] = total;
   }
   __syncthreads();
   for (int r = tid; r < U; r += 1024) {
     const int e = by_rank[r], c = cnt[e], first = cur[e];
-    const int step = wide ? 16 * wt_tiles(c, wide) : UNIT_PAIRS;
-    for (int u = 0; u * step < c; u++) units[rank_base[r] + u] = int4{e, first + u * step, min(step, c - u * step), 0};
+    for (int u = 0; u * UNIT_PAIRS < c; u++)
+      units[rank_base[r] + u] = int4{e, first + u * UNIT_PAIRS, min(UNIT_PAIRS, c - u * UNIT_PAIRS), 0};
   }
   __syncthreads();
   for (int p = tid; p < P; p += 1024) {
@@ -153,8 +151,8 @@ D3_INLINE void group_pairs(const int64_t* ids, int P, int E, int* counts, int* o
 }
 
 __global__ void __launch_bounds__(1024) group_kernel(const int64_t* ids, int P, int E, int* counts, int* offsets,
-                                                     int* perm, int4* units, int* meta, int wide) {
-  group_pairs(ids, P, E, counts, offsets, perm, units, meta, nullptr, wide);
+                                                     int* perm, int4* units, int* meta) {
+  group_pairs(ids, P, E, counts, offsets, perm, units, meta);
 }
 
 // One row of x (bf16, H columns; lane l holds columns 512 c + 8 l .. + 7 in xr[c]) quantized per row: codes in the
@@ -359,7 +357,8 @@ template <int F, int H, int I, int MODE> struct Geometry {
 
 template <int F, int SW> struct Weights {
   Raw<F> raw[2][SW];
-  float rs[2][4];  // I8 / F8: the accumulator rows' scales, per tile
+  float rs[F == FMT_F8 ? 2 : 1][4];  // F8: the accumulator rows' scales, per tile
+  float ers[2];                      // I8: the scales of the rows whose sums this thread completes in the epilogue
 };
 
 // one lane's 32 activation bytes of step `st`
@@ -391,9 +390,18 @@ D3_INLINE void load_weights(Weights<F, Geometry<F, H, I, MODE>::SW>& wt, const P
     const uint8_t* row = bank + (row0 + (lane & 15)) * G::RB;
 #pragma unroll
     for (int j = 0; j < G::SW; j++) load_step<F>(wt.raw[t][j], row, ks * G::SW + j, q);
-    if constexpr (!group_scaled(F)) {
+    if constexpr (F == FMT_F8) {
 #pragma unroll
       for (int i = 0; i < 4; i++) wt.rs[t][i] = bf16_to_f32(sb[row0 + 4 * q + i]);
+    }
+  }
+  if constexpr (F == FMT_I8) {
+    const int tid = threadIdx.x;
+    if constexpr (MODE == 0) {
+#pragma unroll
+      for (int t = 0; t < 2; t++) wt.ers[t] = bf16_to_f32(sb[tile_row0<F, H, I, MODE>(a, e, it, t) + (tid & 15)]);
+    } else {
+      wt.ers[0] = bf16_to_f32(sb[tile_row0<F, H, I, MODE>(a, e, it, 0) + (tid & 63)]);
     }
   }
 }
@@ -406,13 +414,13 @@ D3_INLINE void load_weights(Weights<F, Geometry<F, H, I, MODE>::SW>& wt, const P
 // epilogue and barriers: 164.6 / 164.3 us against 167.8 / 167.7. (Group-scaled weights kept two workgroups per CU
 // that way: W4A8 128.2 against 125.8.) Activation rows are read without a branch (columns past the unit's pairs
 // read its first pair and their products are never stored). colv / colp: per column (pair) of a tile, its epilogue
-// scale and (down) its pair index, staged in LDS by wave 0; rowv (int8): the item's row scales.
+// scale and (down) its pair index, staged in LDS by wave 0.
 constexpr bool late_weights(int F) { return !group_scaled(F); }
 template <int F, int H, int I, int MODE>
 D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
                             const Weights<F, Geometry<F, H, I, MODE>::SW>& wt, int4 unit_n, int4 unit, int it,
                             int c0, const float* gs, float (*part)[Geometry<F, H, I, MODE>::KS][16][17], float* colv,
-                            int* colp, float* rowv, int& pr, Weights<F, Geometry<F, H, I, MODE>::SW>* next_wt, int it_n) {
+                            int* colp, int& pr, Weights<F, Geometry<F, H, I, MODE>::SW>* next_wt, int it_n) {
   using G = Geometry<F, H, I, MODE>;
   constexpr int SW = G::SW, KS = G::KS, K = G::K, STEPS = K / 128;
   constexpr int SHIFT = unpack_shift(F);
@@ -457,15 +465,11 @@ D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
 #pragma unroll
       for (int i = 0; i < 4; i++) y[i] = acc[i] * wt.rs[t][i];
     } else if constexpr (F == FMT_I8) {
-      // the slices' int32 sums meet exactly; the row scale comes after (in LDS, as its bits)
+      // the slices' int32 sums meet exactly (in LDS as their bits); the row scale comes after
       i32x4 acc = {0, 0, 0, 0};
 #pragma unroll
       for (int j = 0; j < SW; j++) acc = step_i8<F>(wt.raw[t][j], lo[j], hi[j], acc);
       y = __builtin_bit_cast(f32x4, acc);
-      if (ks == 0 && c0 == 0 && col == 0) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) rowv[16 * (2 * tp + t) + 4 * q + i] = wt.rs[t][i];
-      }
     } else {
       const float* g = gs + (2 * tp + t) * 16 * STEPS;
       f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -480,6 +484,7 @@ D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
 #pragma unroll
     for (int i = 0; i < 4; i++) part[2 * tp + t][ks][4 * q + i][col] = y[i];
   }
+  const float ers0 = wt.ers[0], ers1 = wt.ers[1];  // before the next item's come
   if (next_wt) load_weights<F, H, I, MODE>(*next_wt, a, unit_n.x, it_n, tp, ks, lane);
   __syncthreads();
   if constexpr (MODE == 0) {
@@ -494,8 +499,8 @@ D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
           g += __float_as_int(part[0][k2][u][j]);
           up += __float_as_int(part[1][k2][u][j]);
         }
-        gv = (float)g * rowv[u];
-        uv = (float)up * rowv[16 + u];
+        gv = (float)g * ers0;
+        uv = (float)up * ers1;
       } else {
 #pragma unroll
         for (int k2 = 0; k2 < KS; k2++) {
@@ -519,7 +524,7 @@ D3_INLINE void compute_tile(const PrefillArgs& a, const int* __restrict__ perm,
           int d = 0;
 #pragma unroll
           for (int k2 = 0; k2 < KS; k2++) d += __float_as_int(part[r >> 4][k2][r & 15][j]);
-          v = (float)d * rowv[r];
+          v = (float)d * ers0;
         } else {
 #pragma unroll
           for (int k2 = 0; k2 < KS; k2++) v += part[r >> 4][k2][r & 15][j];
@@ -536,7 +541,7 @@ template <int F, int H, int I, int MODE>
 D3_INLINE void compute_item(const PrefillArgs& a, const int* __restrict__ perm,
                             Weights<F, Geometry<F, H, I, MODE>::SW>& wt, int4 unit_n, int4 unit, int it,
                             float* gs, float (*part)[Geometry<F, H, I, MODE>::KS][16][17], float* colv, int* colp,
-                            float* rowv, int& pr, bool more, int it_n) {
+                            int& pr, bool more, int it_n) {
   using G = Geometry<F, H, I, MODE>;
   constexpr int STEPS = G::K / 128;
   const int tid = threadIdx.x;
@@ -552,12 +557,12 @@ D3_INLINE void compute_item(const PrefillArgs& a, const int* __restrict__ perm,
   const int last = (unit.z - 1) & ~15;
   if constexpr (late_weights(F)) {
     for (int c0 = 0; c0 < last; c0 += 16)
-      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, rowv, pr, nullptr, 0);
-    compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, last, gs, part, colv, colp, rowv, pr, more ? &wt : nullptr,
+      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, pr, nullptr, 0);
+    compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, last, gs, part, colv, colp, pr, more ? &wt : nullptr,
                                 it_n);
   } else {
     for (int c0 = 0; c0 <= last; c0 += 16)
-      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, rowv, pr, nullptr, 0);
+      compute_tile<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, c0, gs, part, colv, colp, pr, nullptr, 0);
   }
 }
 
@@ -571,7 +576,6 @@ __global__ void __launch_bounds__(256) grouped_kernel(PrefillArgs a, const int4*
   __shared__ float gs[group_scaled(F) ? G::TILES * 16 * (G::K / 128) : 1];
   __shared__ float colv[16];
   __shared__ int colp[16];
-  __shared__ float rowv[F == FMT_I8 ? G::TILES * 16 : 1];
   const int n_items = meta[0] * G::PER_EXPERT;
   int i = blockIdx.x;
   if (i >= n_items) return;
@@ -592,7 +596,7 @@ __global__ void __launch_bounds__(256) grouped_kernel(PrefillArgs a, const int4*
     const bool more = in < n_items;
     const int4 unit_n = units[(more ? in : i) / G::PER_EXPERT];
     const int it_n = (more ? in : i) % G::PER_EXPERT;
-    compute_item<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, gs, part, colv, colp, rowv, pr, more, it_n);
+    compute_item<F, H, I, MODE>(a, perm, wt, unit_n, unit, it, gs, part, colv, colp, pr, more, it_n);
     if (!more) break;
     i = in;
     rnd++;
@@ -617,7 +621,7 @@ __global__ void __launch_bounds__(256) reduce_kernel(const float* parts, int T, 
 
 // ------------------------------------------------------------------------------------------------------- host side
 struct Layout {
-  size_t ids, weights, counts, offsets, perm, units, meta, xq, xs, h, hq, hs, parts, total;
+  size_t ids, weights, counts, offsets, perm, units, meta, hist, xq, xs, h, hq, hs, parts, total;
 };
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 Layout layout(int64_t T, int64_t k, int64_t H, int64_t I, int64_t E) {
@@ -632,6 +636,7 @@ Layout layout(int64_t T, int64_t k, int64_t H, int64_t I, int64_t E) {
   L.perm = take(P * 4);
   L.units = take((E + P / UNIT_PAIRS + 1) * 16);
   L.meta = take(16);
+  L.hist = take((int64_t)PG_BLOCKS * E * 4);
   L.xq = take(T * H);
   L.xs = take(T * 4);
   L.h = take(P * I * 4);
@@ -807,10 +812,23 @@ int d3_moe_a8_prefill(const d3_moe_a8_prefill_desc* d, void* stream) {
       default: route_quant<FMT_F8>(*d, ids, weights, xq, xs, s); break;
     }
   }
-  if (!small)
+  if (wide_fits(*d)) {
+    PromptGroups g;
+    g.ids = ids;
+    g.P = P;
+    g.E = d->E;
+    g.clamp = true;
+    g.perm = (int*)(ws + L.perm);
+    g.passes = (int4*)(ws + L.units);
+    g.count = (int*)(ws + L.meta);
+    g.cap = std::min(d->E, P) + P / (16 * a8_wide_tiles(d->format));
+    g.tiles = a8_wide_tiles(d->format);
+    g.hist = (int*)(ws + L.hist);
+    launch_prompt_hist(g, s);
+    launch_prompt_scatter(g, s);
+  } else if (!small)
     hipLaunchKernelGGL(group_kernel, dim3(1), dim3(1024), 0, s, (const int64_t*)ids, P, d->E, (int*)(ws + L.counts),
-                       (int*)(ws + L.offsets), (int*)(ws + L.perm), (int4*)(ws + L.units), (int*)(ws + L.meta),
-                       wide_fits(*d) ? a8_wide_tiles(d->format) : 0);
+                       (int*)(ws + L.offsets), (int*)(ws + L.perm), (int4*)(ws + L.units), (int*)(ws + L.meta));
   PrefillArgs pa;
   pa.ids = ids;
   pa.weights = weights;

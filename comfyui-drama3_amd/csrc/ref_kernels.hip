@@ -16,7 +16,7 @@
 // the codes on the int8 cores against the rows as three int8 planes with a power-of-two scale (grouped_i8_kernel),
 // FP8 on the bf16 cores against exact bf16 planes (grouped_fp8_kernel), each weight read once per 32-row pass.
 #include "ref_common.hpp"
-#include "wide_tile.hpp"
+#include "prompt_group.hpp"
 #include "../../include/drama3_moe.h"
 
 #include <algorithm>
@@ -586,12 +586,9 @@ __global__ void __launch_bounds__(256) grouped_plan_kernel(const int* groups, in
 // after every group, inverse -1. With `work`, the same workgroup also plans the grouped products' passes over the
 // groups (grouped_plan_kernel's plan, from the counts it holds), so that takes no launch of its own.
 constexpr int GROUPS_MAX_E = 1024;
-// With `wide`, the passes of the wide products instead (pass_cap places of (expert, first row, rows, 0) after the count
-// at wide[0], at most WIDE_TILES 16-row tiles each): the passes with most tiles first, an expert's passes together.
 D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* order, int* inverse, int* groups,
-                                  int* work, int cap, int* wide, int wide_cap) {
+                                  int* work, int cap) {
   __shared__ int count[GROUPS_MAX_E + 1], cursor[GROUPS_MAX_E + 1], wave_total[16], pcount[8], pcursor[8];
-  static_assert(WIDE_TILES <= 8, "a bucket of pcount per number of tiles");
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int e = tid; e <= E; e += 1024) count[e] = 0;
   if (tid < 8) pcount[tid] = 0;
@@ -615,7 +612,7 @@ D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* ord
   for (int i = 0; i < w; i++) before += wave_total[i];
   const int first = before + incl - v;
   if (tid <= E) cursor[tid] = first;
-  if (groups && tid < E) {
+  if (tid < E) {
     int* gp = groups + 5 * tid;
     gp[0] = tid;
     gp[1] = tid;
@@ -635,25 +632,6 @@ D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* ord
     __syncthreads();
     if (tid < E) plan_put(tid, first, v, P, pcursor, work, cap);
   }
-  if (wide) {  // bucket b: passes of WIDE_TILES - b tiles
-    const int np = tid < E ? wt_passes(v, WIDE_TILES) : 0, tiles = wt_tiles(v, WIDE_TILES);
-    if (np) atomicAdd(&pcount[WIDE_TILES - tiles], np);
-    __syncthreads();
-    if (tid == 0) {
-      int at = 0;
-      for (int b = 0; b < WIDE_TILES; b++) {
-        pcursor[b] = at;
-        at += pcount[b];
-      }
-      wide[0] = min(at, wide_cap);
-    }
-    __syncthreads();
-    if (np) {
-      const int at = atomicAdd(&pcursor[WIDE_TILES - tiles], np), step = 16 * tiles;
-      for (int i = 0; i < np && at + i < wide_cap; i++)
-        ((int4*)(wide + 4))[at + i] = int4{tid, first + i * step, min(step, v - i * step), 0};
-    }
-  }
   __syncthreads();
   for (int p = tid; p < P; p += 1024) {
     const int64_t e = ids[p];
@@ -665,9 +643,8 @@ D3_INLINE void expert_groups_body(const int64_t* ids, int P, int E, int64_t* ord
 }
 
 __global__ void __launch_bounds__(1024) expert_groups_kernel(const int64_t* ids, int P, int E, int64_t* order,
-                                                             int* inverse, int* groups, int* work, int cap,
-                                                             int* wide, int wide_cap) {
-  expert_groups_body(ids, P, E, order, inverse, groups, work, cap, wide, wide_cap);
+                                                             int* inverse, int* groups, int* work, int cap) {
+  expert_groups_body(ids, P, E, order, inverse, groups, work, cap);
 }
 
 // columns c0 .. c0 + 3 of row `row` of x as float (SRC as for prep_planes_kernel)
@@ -792,18 +769,25 @@ __global__ void __launch_bounds__(256) prep_i8_kernel(const void* x, const int64
 }
 
 // The grouping (workgroup 0, expert_groups_kernel's) and the token rows' int8 planes (prep_i8_kernel's, 4 rows per
-// later workgroup) in one launch: neither waits for the other, so the planes cost no launch of their own.
-template <int SRC, bool ROT>
+// later workgroup) in one launch: neither waits for the other, so the planes cost no launch of their own. WIDE: the
+// first workgroups count a long prompt's blocks of pairs instead (prompt_group.hpp).
+template <int SRC, bool ROT, bool WIDE>
 __global__ void __launch_bounds__(1024) groups_prep_kernel(const int64_t* ids, int P, int E, int64_t* order,
                                                            int* inverse, int* groups, int* work, int cap,
-                                                           int* wide, int wide_cap, const void* x, int T, int K,
+                                                           PromptGroups pg, const void* x, int T, int K,
                                                            int8_t* planes, float* scales) {
-  if (blockIdx.x == 0) {
-    expert_groups_body(ids, P, E, order, inverse, groups, work, cap, wide, wide_cap);
+  const int before = WIDE ? pg_blocks(pg.P) : 1;
+  if ((int)blockIdx.x < before) {
+    if constexpr (WIDE) {
+      __shared__ int cnt[PG_MAX_E];
+      prompt_hist_block(pg, blockIdx.x, cnt);
+    } else {
+      expert_groups_body(ids, P, E, order, inverse, groups, work, cap);
+    }
     return;
   }
   __shared__ uint32_t wmax[4][4];
-  const int tid = threadIdx.x, r = tid >> 8, p = 4 * ((int)blockIdx.x - 1) + r;
+  const int tid = threadIdx.x, r = tid >> 8, p = 4 * ((int)blockIdx.x - before) + r;
   prep_i8_row<SRC, ROT>(x, nullptr, 1, K, planes, (int64_t)T * K, scales, p, p < T, (tid >> 6) & 3, tid & 63,
                         (tid & 255) == 0, wmax[r]);
 }
@@ -2149,22 +2133,26 @@ static int check_rows(const char* what, int64_t plane, int32_t K, const int64_t*
 }
 
 static int groups_prep(const char* what, const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse,
-                       int32_t* groups, int32_t* work, int cap, int32_t* wide, int wide_cap, int32_t mode,
-                       int32_t rotate, const void* x, int32_t T, int32_t K, void* planes, float* scales,
-                       void* stream) {
+                       int32_t* groups, int32_t* work, int cap, const PromptGroups* pg, int32_t mode, int32_t rotate,
+                       const void* x, int32_t T, int32_t K, void* planes, float* scales, void* stream) {
   if (P > 0 && (!ids || !order || !inverse)) return fail(std::string(what) + ": null pointer");
   if (T > 0 && (!x || !planes || !scales)) return fail(std::string(what) + ": null pointer");
   if (T < 0 || (mode != 0 && mode != 1) || !supported_k(K))
     return fail(std::string(what) + ": T >= 0, mode 0 (float32 rows) or 1 (bf16 rows), K in {256..2048}");
   const hipStream_t s = (hipStream_t)stream;
-  const dim3 grid(1 + (T + 3) / 4);
+  const dim3 grid((pg ? pg_blocks(P) : 1) + (T + 3) / 4);
   int8_t* pl = (int8_t*)planes;
-#define D3_GP(M, R) hipLaunchKernelGGL((groups_prep_kernel<M, R>), grid, dim3(1024), 0, s, ids, P, E, order, inverse, groups, work, cap, wide, wide_cap, x, T, K, pl, scales)
+#define D3_GP(M, R)                                                                                                  \
+  if (pg) hipLaunchKernelGGL((groups_prep_kernel<M, R, true>), grid, dim3(1024), 0, s, ids, P, E, order, inverse,    \
+                             groups, work, cap, *pg, x, T, K, pl, scales);                                           \
+  else hipLaunchKernelGGL((groups_prep_kernel<M, R, false>), grid, dim3(1024), 0, s, ids, P, E, order, inverse,      \
+                          groups, work, cap, PromptGroups{}, x, T, K, pl, scales);                                   \
+  break
   switch (mode * 2 + (rotate ? 1 : 0)) {
-    case 0: D3_GP(0, false); break;
-    case 1: D3_GP(0, true); break;
-    case 2: D3_GP(1, false); break;
-    default: D3_GP(1, true); break;
+    case 0: D3_GP(0, false);
+    case 1: D3_GP(0, true);
+    case 2: D3_GP(1, false);
+    default: D3_GP(1, true);
   }
 #undef D3_GP
   return done(what);
@@ -2178,18 +2166,53 @@ int d3_expert_groups_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* 
   const int64_t need = d3_grouped_mfma_work_ints(E, P);
   if (work_ints < need) return fail("d3_expert_groups_prep_i8: work holds fewer than d3_grouped_mfma_work_ints ints");
   return groups_prep("d3_expert_groups_prep_i8", ids, P, E, order, inverse, groups, work, (int)((need - 2) / 2),
-                     nullptr, 0, mode, rotate, x, T, K, planes, scales, stream);
+                     nullptr, mode, rotate, x, T, K, planes, scales, stream);
+}
+
+// the grouping of a resident prompt: passes holds the count, the list, then the blocks' counts
+static int prompt_groups_of(const char* what, const int64_t* ids, int32_t P, int32_t E, int64_t* order,
+                            int32_t* inverse, int32_t* passes, int64_t pass_ints, PromptGroups& g) {
+  if (!ids || !order || !inverse || !passes) return fail(std::string(what) + ": null pointer");
+  if (P < 1 || E < 1 || E > PG_MAX_E) return fail(std::string(what) + ": 1 <= E <= 1024, P >= 1");
+  if (pass_ints < d3_prompt_pass_ints(E, P)) return fail(std::string(what) + ": passes holds fewer than d3_prompt_pass_ints ints");
+  g.ids = ids;
+  g.P = P;
+  g.E = E;
+  g.clamp = false;
+  g.order = order;
+  g.inverse = inverse;
+  g.count = passes;
+  g.passes = (int4*)(passes + 4);
+  g.tiles = WIDE_TILES;
+  g.cap = P / (16 * WIDE_TILES) + std::min(E, P);
+  g.hist = passes + 4 + 4 * (int64_t)g.cap;
+  return 0;
+}
+
+int64_t d3_prompt_pass_ints(int32_t E, int64_t P) {
+  if (E < 1 || P < 0) return -1;
+  return 4 + 4 * (P / (16 * WIDE_TILES) + std::min<int64_t>(E, P)) + (int64_t)PG_BLOCKS * E;
 }
 
 int d3_prompt_prep_i8(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse, int32_t* passes,
                       int64_t pass_ints, int32_t mode, int32_t rotate, const void* x, int32_t T, int32_t K,
                       void* planes, float* scales, void* stream) {
-  if (!passes) return fail("d3_prompt_prep_i8: null pointer");
-  if (P < 0 || E < 1 || E > GROUPS_MAX_E) return fail("d3_prompt_prep_i8: 1 <= E <= 1024, P >= 0");
-  const int64_t need = d3_prompt_pass_ints(E, P);
-  if (pass_ints < need) return fail("d3_prompt_prep_i8: passes holds fewer than d3_prompt_pass_ints ints");
-  return groups_prep("d3_prompt_prep_i8", ids, P, E, order, inverse, nullptr, nullptr, 0, passes, (int)((need - 4) / 4),
-                     mode, rotate, x, T, K, planes, scales, stream);
+  PromptGroups g;
+  if (const int e = prompt_groups_of("d3_prompt_prep_i8", ids, P, E, order, inverse, passes, pass_ints, g)) return e;
+  if (const int e = groups_prep("d3_prompt_prep_i8", ids, P, E, order, inverse, nullptr, nullptr, 0, &g, mode, rotate, x,
+                                T, K, planes, scales, stream))
+    return e;
+  launch_prompt_scatter(g, (hipStream_t)stream);
+  return done("d3_prompt_prep_i8");
+}
+
+int d3_prompt_groups(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse, int32_t* passes,
+                     int64_t pass_ints, void* stream) {
+  PromptGroups g;
+  if (const int e = prompt_groups_of("d3_prompt_groups", ids, P, E, order, inverse, passes, pass_ints, g)) return e;
+  launch_prompt_hist(g, (hipStream_t)stream);
+  launch_prompt_scatter(g, (hipStream_t)stream);
+  return done("d3_prompt_groups");
 }
 
 int d3_grouped_fp8(const void* planes, int32_t n_planes, int64_t plane, const int64_t* order, int32_t k,
@@ -2238,19 +2261,8 @@ int d3_expert_groups(const int64_t* ids, int32_t P, int32_t E, int64_t* order, i
     cap = (int)((need - 2) / 2);
   }
   hipLaunchKernelGGL(expert_groups_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, P, E, order, inverse,
-                     groups, work, cap, nullptr, 0);
+                     groups, work, cap);
   return done("d3_expert_groups");
-}
-
-int d3_prompt_groups(const int64_t* ids, int32_t P, int32_t E, int64_t* order, int32_t* inverse, int32_t* passes,
-                     int64_t pass_ints, void* stream) {
-  if (!passes || (P > 0 && (!ids || !order || !inverse))) return fail("d3_prompt_groups: null pointer");
-  if (P < 0 || E < 1 || E > GROUPS_MAX_E) return fail("d3_prompt_groups: 1 <= E <= 1024, P >= 0");
-  const int64_t need = d3_prompt_pass_ints(E, P);
-  if (pass_ints < need) return fail("d3_prompt_groups: passes holds fewer than d3_prompt_pass_ints ints");
-  hipLaunchKernelGGL(expert_groups_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, P, E, order, inverse,
-                     nullptr, nullptr, 0, passes, (int)((need - 4) / 4));
-  return done("d3_prompt_groups");
 }
 
 int d3_prep_planes(int32_t mode, int32_t rotate, int32_t n_planes, const void* x, const int64_t* order, int32_t k,

@@ -300,11 +300,6 @@ using namespace d3;
 
 extern "C" {
 
-int64_t d3_prompt_pass_ints(int32_t E, int64_t P) {
-  if (E < 1 || P < 0) return -1;
-  return 4 + 4 * (P / (16 * WI_TILES) + std::min<int64_t>(E, P));
-}
-
 int d3_prompt_i8(int32_t kind, const void* planes, const float* scales, int64_t plane, const int64_t* order, int32_t k,
                  int32_t rows, const int32_t* passes, int64_t pass_ints, int32_t E, const void* w, const void* s,
                  const float* c, const float* codebook, float* out, int32_t N, int32_t K, int32_t swiglu, void* stream) {
@@ -335,7 +330,7 @@ int d3_prompt_i8(int32_t kind, const void* planes, const float* scales, int64_t 
   a.out = out;
   a.N = N;
   a.K = K;
-  const int cap = (int)((d3_prompt_pass_ints(E, rows) - 4) / 4);
+  const int cap = rows / (16 * WI_TILES) + std::min(E, rows);
   const dim3 grid((unsigned)(wt_places(cap) * (N / WT_N)));
   const hipStream_t st = (hipStream_t)stream;
 #define D3_WIDE(KD)                                                                                                  \

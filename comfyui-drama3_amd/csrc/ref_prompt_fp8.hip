@@ -234,7 +234,7 @@ extern "C" int d3_prompt_fp8(const void* planes, int32_t n_planes, int64_t plane
     return fail("d3_prompt_fp8: 1 <= rows (<= plane / K without order), k >= 1 with order");
   if (((uintptr_t)planes | (uintptr_t)w) & 15) return fail("d3_prompt_fp8: planes and weights at 16-byte alignment");
   if (pass_ints < d3_prompt_pass_ints(E, rows)) return fail("d3_prompt_fp8: passes holds fewer than d3_prompt_pass_ints ints");
-  const int cap = (int)((d3_prompt_pass_ints(E, rows) - 4) / 4);
+  const int cap = rows / (16 * WIDE_TILES) + std::min(E, rows);
   WideF8Args a;
   a.xs = (const uint8_t*)planes;
   a.plane = 2 * plane;

@@ -296,8 +296,9 @@ int d3_grouped_i8(int32_t kind, const void* planes, const float* scales, int64_t
 
 /* The same products for a long prompt on banks held whole on the GPU (expert e's N rows at e * N; offload.py:138-149
  * with no slot cache): passes of up to 96 rows against 256 weight rows per workgroup. d3_prompt_prep_i8 does what
- * d3_expert_groups_prep_i8 does, with the passes as its plan: passes [4 + 4 n] int32 (>= d3_prompt_pass_ints(E, P)),
- * passes[0] their number, then (expert, first row in order, rows, 0) each. d3_prompt_i8 runs one bank (w, s, c: the
+ * d3_expert_groups_prep_i8 does, with the passes as its plan: passes int32 [>= d3_prompt_pass_ints(E, P)],
+ * passes[0] their number, then (expert, first row in order, rows, 0) each from passes[4] (and the blocks' counts that
+ * the grouping's two launches exchange); P >= 1. d3_prompt_i8 runs one bank (w, s, c: the
  * expert fields, as host_w, host_s, host_c of d3_grouped_i8) over them, out [rows, N] float32 =
  * scale * (S * (A0 + (A1 + A2 / 254) / 254)) as d3_grouped_i8, each step of the sum over the planes rounded once.
  * With swiglu the bank's rows are N / 2 gate rows, then N / 2 up rows, and out [rows, N / 2] = SiLU(gate) * up.

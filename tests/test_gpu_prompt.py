@@ -16,6 +16,35 @@ pytestmark = pytest.mark.gpu
 COUNTS = [0, 1, 15, 16, 17, 95, 96, 97, 193, 240, 50]
 
 
+@pytest.mark.parametrize("E, P", [(1, 1), (7, 1023), (128, 1025), (256, 30011), (1024, 70000), (100, 131072 + 5)])
+def test_prompt_groups(E, P):
+    """The grouping over many workgroups, from one pair to more than 64 blocks of 1024 of them, some ids outside the
+    experts: every pair once, the experts in ascending order, inverse the pairs' places (-1 and after every group for
+    an id outside), and passes that cover each expert's places in runs of at most 96, those of most tiles first."""
+    rng = np.random.default_rng(E)
+    ids = rng.integers(0, E, P)
+    ids[rng.random(P) < 0.3] = E // 2
+    bad = rng.random(P) < 0.01
+    ids[bad] = rng.choice([-1, E, E + 5, -2 ** 40, 2 ** 40], size=int(bad.sum()))
+    order, inverse, passes = (t.cpu().numpy() for t in kernels.prompt_groups(dev(ids.astype(np.int64)).view(-1, 1), E))
+    assert np.array_equal(np.sort(order), np.arange(P))
+    valid = (ids >= 0) & (ids < E)
+    n = int(valid.sum())
+    assert np.array_equal(ids[order[:n]], np.sort(ids[valid])) and not valid[order[n:]].any()
+    assert np.array_equal(inverse[order[:n]], np.arange(n)) and np.all(inverse[~valid] == -1)
+    listed = passes[4:4 + 4 * passes[0]].reshape(-1, 4)
+    tiles = (listed[:, 2] + 15) // 16
+    assert np.all(listed[:, 2] >= 1) and np.all(tiles <= 6)
+    counts = np.bincount(ids[valid], minlength=E)
+    first = np.cumsum(counts) - counts
+    for e in np.unique(ids[valid]):
+        own = listed[listed[:, 0] == e]
+        own = own[np.argsort(own[:, 1])]
+        assert own[0, 1] == first[e] and np.array_equal(own[1:, 1], own[:-1, 1] + own[:-1, 2])
+        assert own[:, 2].sum() == counts[e] and len(set(((own[:-1, 2] + 15) // 16).tolist())) <= 1
+    assert set(listed[:, 0].tolist()) == set(np.unique(ids[valid]).tolist())
+
+
 @pytest.mark.parametrize("K, N", [(256, 512), (2048, 256), (768, 1024)])
 @pytest.mark.parametrize("kind", ["int8", "w4", "w6"])
 def test_prompt_products_match_the_32_row_products(kind, K, N):
