@@ -3,10 +3,10 @@
 // times over for the first bank. That suits experts with a few rows; with hundreds, this kernel's 256 x 256 tiles read
 // both operands from L2 an eighth as often and run a wave's 64 x 128 tile from LDS (128 accumulators a lane, two waves
 // per SIMD).
-// Measured, top-8 of 128 experts (FFN 768), first / second bank's products: int8, 4096 rows 512 / 260 us before, 199 /
-// 148 here (8192 rows, Zipf routing: the layer 1701 / 747); FP8 the same, W4 234 / 156 (808 / 497), W6 the layer 885 /
-// 553. At 4096 rows the banks' and results' bytes take about 105 us of each at the rate a copy reaches and the int8
-// products 100 and 50: they overlap within a workgroup, but its first loads and its stores do not.
+// Measured, 4096 rows, top-8 of 128 experts (FFN 768), first / second bank's products: int8 512 / 260 us before, 199 /
+// 147 here, FP8 240 / 181; the layer: int8 874 / 415, FP8 879 / 489, W4 807 / 448, W6 882 / 499 (8192 rows, Zipf
+// routing: int8 1703 / 698). The banks' and results' bytes take about 105 us of each int8 product at the rate a copy
+// reaches and the products 100 and 50: they overlap within a workgroup, but its first loads and its stores do not.
 #include "a8_wide.hpp"
 #include "formats.hpp"
 

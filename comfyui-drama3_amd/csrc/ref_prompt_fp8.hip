@@ -6,8 +6,8 @@
 // to 96 rows: the weights lie in LDS as their e4m3 bytes, 128 columns at a time, and each wave widens its 64 rows'
 // operands as it reads them (two codes an instruction); the rows lie there as bf16, in tiles of 64 columns. A lane's
 // columns of such a tile are 16 (l >> 4) .. + 15, in two steps of 8, weights and rows alike.
-// Measured us per layer before / here: 8192 rows, top-8 of 128 experts (FFN 768, Zipf routing) 2275 / 1413, 2391 rows of
-// 256 experts (FFN 512) 636 / 425.
+// Measured us per layer before / here: 8192 rows, top-8 of 128 experts (FFN 768, Zipf routing) 2266 / 1331 (first bank's
+// products 546, second's 731: three planes), 2391 rows of 256 experts (FFN 512) 625 / 402.
 #include "ref_common.hpp"
 #include "wide_tile.hpp"
 #include "../../include/drama3_moe.h"
