@@ -384,7 +384,11 @@ def _wide_pairs(x, topk_idx, banks, rows, kind, codebooks, num_experts):
     top_k, width, inner = topk_idx.shape[1], x.shape[1], rows[0] // 2
     if kind == "fp8":
         order, inverse, passes = kernels.prompt_groups(topk_idx, num_experts)
-        planes = x.contiguous().view(1, -1) if x.dtype == torch.bfloat16 else kernels.prep_planes(x, False)
+        if x.dtype == torch.bfloat16:   # bf16 rows are their own one plane, which the copies to LDS want 16-byte aligned
+            x = x.contiguous()
+            planes = (x if x.data_ptr() % 16 == 0 else x.clone()).view(1, -1)
+        else:
+            planes = kernels.prep_planes(x, False)
         P = order.shape[0]
         hidden = kernels.prompt_fp8(planes, P, width, passes, num_experts, banks[0], rows[0], order, top_k, swiglu=True)
         planes = kernels.prep_planes(hidden, False)

@@ -169,3 +169,19 @@ def test_prompt_path_equals_the_32_row_path_and_replays(kind, monkeypatch):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.view(torch.int16), run().view(torch.int16))
+
+
+def test_prompt_fp8_rows_at_any_storage_offset():
+    """Contiguous bf16 rows that start one element into their storage (bf16 rows are FP8's plane as they are): the same
+    result as the aligned rows, bit for bit, from as many rows as the wide products take."""
+    rng = np.random.default_rng(40)
+    E, T, k, H, I = 4, 97, 2, 256, 256
+    banks = [fields_on(b) for b in (_bank("fp8", rng, E, 2 * I, H), _bank("fp8", rng, E, H, I))]
+    idx = dev(zipf_topk(rng, T, E, k).astype(np.int64))
+    w = dev(rng.dirichlet(np.ones(k), T).astype(np.float32))
+    x = dev(rng.standard_normal((T, H)).astype(np.float32)).to(torch.bfloat16)
+    offset = torch.empty(T * H + 1, dtype=torch.bfloat16, device=DEV)[1:].view(T, H).copy_(x)
+    assert offset.is_contiguous() and offset.data_ptr() % 16 == 2
+    assert kernels.prompt_wide_fits("fp8", banks, (2 * I, H), T * k, E, H)
+    got, want = (offload.resident_prefill(v, idx, w, banks, (2 * I, H), "fp8", (None, None), E) for v in (offset, x))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
