@@ -19,16 +19,17 @@ D3_INLINE uint32_t lds_address(const void* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
 }
 // 16 bytes per lane from base + off (the lane's own) into LDS at lds + 16 * lane (lds uniform over the wave), without
-// passing through registers. The compiler does not count these loads: dma_wait() before the barrier that hands them to
-// the other waves.
+// passing through registers. The instruction takes lds from m0: as an operand of the statement, so that the compiler
+// knows what m0 holds after it. The compiler does not count these loads: dma_wait() before the barrier that hands them
+// to the other waves.
 D3_INLINE void dma16(uint32_t lds, const void* base, uint32_t off) {
   // (both uniform already; said again for the compiler, which may keep a loop's pointers in vector registers)
   const uint64_t at = (uint64_t)base;
   const uint64_t sbase = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at) |
                          (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32;
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :
-               : "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(off), "s"(sbase)
+               : "{m0}"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(off), "s"(sbase)
                : "memory");
 }
 D3_INLINE void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
