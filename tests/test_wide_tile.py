@@ -27,17 +27,43 @@ def _build():
     return module
 
 
-def test_dma16_tells_the_compiler_that_it_writes_m0(tmp_path):
-    """A value that the compiler keeps in m0 on both sides of a copy to LDS, whose LDS address the copy puts there: m0
-    is set again before the second use."""
+def _assembly(tmp_path, source):
     build = _build()
     if not build.HIPCC.exists():
         pytest.skip("no hipcc")
     src, out = tmp_path / "k.hip", tmp_path / "k.s"
-    src.write_text(KERNEL)
+    src.write_text(source)
     subprocess.run([str(build.HIPCC), *build.FLAGS, f"-I{CSRC}", "--cuda-device-only", "-S", str(src), "-o", str(out)],
                    check=True, capture_output=True)
-    text = out.read_text()
+    return out.read_text()
+
+
+def test_dma16_tells_the_compiler_that_it_writes_m0(tmp_path):
+    """A value that the compiler keeps in m0 on both sides of a copy to LDS, whose LDS address the copy puts there: m0
+    is set again before the second use."""
+    text = _assembly(tmp_path, KERNEL)
     copy, second = text.index("global_load_lds_dwordx4"), text.index("; second use of m0")
     assert text.index("; first use of m0") < copy < second
     assert re.search(r"s_mov_b32 m0, s\d+", text[copy:second])
+
+
+BASE_IN_VECTOR_REGISTERS = """
+#include "wide_tile.hpp"
+__global__ void k(const char* const* bases, const int* lds_at) {
+  __shared__ uint8_t lds[4096];
+  const char* base = bases[threadIdx.x >> 6];
+  d3::dma16(d3::lds_address(lds) + lds_at[threadIdx.x >> 6], base, 16 * (threadIdx.x & 63));
+  d3::dma_wait();
+}
+"""
+
+
+def test_dma16_waits_for_scalar_registers_written_by_vector_instructions(tmp_path):
+    """A base and an LDS address that come from vector registers: five wait states between the last readfirstlane and
+    the copy that reads its result (an instruction is one, s_nop n is n + 1)."""
+    lines = [line.split(";")[0].split() for line in _assembly(tmp_path, BASE_IN_VECTOR_REGISTERS).splitlines()]
+    ops = [line for line in lines if line and not line[0].startswith(".") and not line[0].endswith(":")]
+    copy = next(i for i, op in enumerate(ops) if op[0] == "global_load_lds_dwordx4")
+    reads = [i for i in range(copy) if ops[i][0] == "v_readfirstlane_b32"]
+    assert len(reads) >= 3
+    assert sum(int(op[1]) + 1 if op[0] == "s_nop" else 1 for op in ops[reads[-1] + 1:copy]) >= 5
