@@ -42,6 +42,26 @@ D3_INLINE uint32_t lookup16(i32x4 t, uint32_t sel) {
 
 constexpr float I8_RATIO = 254.0f;  // the int8 planes' ratio
 
+// x / 254 correctly rounded: the remainder of the first quotient by one fused step, its quotient added by another (the
+// same bits as the division for every float x down to 2^-100; the divide instruction sequence takes three times as many)
+D3_INLINE float over_ratio(float x) {
+  constexpr float INV = 1.0f / I8_RATIO;
+  const float q = x * INV;
+  return fmaf(fmaf(-I8_RATIO, q, x), INV, q);
+}
+// SiLU(gate) * up, the product rounded by itself: left to contraction, a kernel that goes on to add it up (a rotation)
+// would take it unrounded, one that stores it rounded, and a row's result would depend on which of them runs it.
+D3_INLINE float silu_up(float gate, float up) {
+#pragma clang fp contract(off)
+  return gate / (1.0f + __expf(-gate)) * up;
+}
+
+// The planes' exact sums of one output in float32, every step rounded once: A0 + (A1 + A2 / 254) / 254. All the int8
+// products end in it, so a row's result does not depend on which of them runs it.
+D3_INLINE float planes_sum(int a0, int a1, int a2) {
+  return (float)a0 + over_ratio((float)a1 + over_ratio((float)a2));
+}
+
 // W4: one 16-code group's int8-grid values as bytes in column order (word d: codes 4d .. 4d + 3) through the
 // group's scale-byte row t of a signed table (build_qtab<true>); lo / hi: the nibble words of codes 0-7 / 8-15
 // (code j's nibble at bits 4 (j & 7))

@@ -661,7 +661,7 @@ template <int SRC> D3_INLINE void load_row4(const void* x, size_t row, int K, in
     const f32x4 gt = *(const f32x4*)(f + c0), up = *(const f32x4*)(f + K + c0);
     const float gg[4] = {gt.x, gt.y, gt.z, gt.w}, uu[4] = {up.x, up.y, up.z, up.w};
 #pragma unroll
-    for (int j = 0; j < 4; j++) v[j] = gg[j] / (1.0f + __expf(-gg[j])) * uu[j];
+    for (int j = 0; j < 4; j++) v[j] = silu_up(gg[j], uu[j]);
   }
 }
 
@@ -1213,10 +1213,8 @@ __global__ void __launch_bounds__(256, 2) grouped_i8_kernel(const int8_t* xs, in
       for (int a = 0; a < RA; a++) {
         f32x4 o;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float mid = (float)acc[a][mt][1][i] + (float)acc[a][mt][2][i] / I8_RATIO;
-          o[i] = es[a][i] * (sx * ((float)acc[a][mt][0][i] + mid / I8_RATIO));
-        }
+        for (int i = 0; i < 4; i++)
+          o[i] = es[a][i] * (sx * planes_sum(acc[a][mt][0][i], acc[a][mt][1][i], acc[a][mt][2][i]));
         *(f32x4*)(out + (size_t)(first + r) * N + nw + 16 * a + 4 * q) = o;
       }
     }

@@ -254,9 +254,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_i8_kernel(WideArgs a) {
       __syncthreads();
     }
 
-    // lane l holds weight rows 64 wn + 16 n + 4 q .. + 3 of the pass's row 16 mt + c; the planes' sums meet in
-    // float32 as A0 + (A1 + A2 / 254) / 254, each step one fused rounding
-    constexpr float INV = 1.0f / I8_RATIO;
+    // lane l holds weight rows 64 wn + 16 n + 4 q .. + 3 of the pass's row 16 mt + c
 #pragma unroll
     for (int j = 0; j < NT; j++) {
       const int r = 16 * (wm + 2 * j) + c;
@@ -268,7 +266,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_i8_kernel(WideArgs a) {
           const f32x4 e = *(const f32x4*)(factors + 64 * wn + 16 * n + 4 * q);
 #pragma unroll
           for (int i = 0; i < 4; i++)
-            v[n][i] = e[i] * (sx * fmaf(fmaf((float)acc[n][j][2][i], INV, (float)acc[n][j][1][i]), INV, (float)acc[n][j][0][i]));
+            v[n][i] = e[i] * (sx * planes_sum(acc[n][j][0][i], acc[n][j][1][i], acc[n][j][2][i]));
         }
         if constexpr (SWIGLU) {
           float* o = a.out + (size_t)(first + r) * (N / 2) + xb * (WT_N / 2) + 32 * wn + 4 * q;
@@ -276,7 +274,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_i8_kernel(WideArgs a) {
           for (int n = 0; n < 2; n++) {
             f32x4 h;
 #pragma unroll
-            for (int i = 0; i < 4; i++) h[i] = v[n][i] / (1.0f + __expf(-v[n][i])) * v[n + 2][i];
+            for (int i = 0; i < 4; i++) h[i] = silu_up(v[n][i], v[n + 2][i]);
             *(f32x4*)(o + 16 * n) = h;
           }
         } else {

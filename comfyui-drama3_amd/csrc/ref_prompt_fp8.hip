@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_fp8_kernel(WideF8Args a) {
           for (int n = 0; n < 2; n++) {
             f32x4 h;
 #pragma unroll
-            for (int i = 0; i < 4; i++) h[i] = acc[j][n][i] / (1.0f + __expf(-acc[j][n][i])) * acc[j][n + 2][i];
+            for (int i = 0; i < 4; i++) h[i] = silu_up(acc[j][n][i], acc[j][n + 2][i]);
             *(f32x4*)(o + 16 * n) = h;
           }
         } else {

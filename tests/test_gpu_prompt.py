@@ -49,9 +49,8 @@ def test_prompt_groups(E, P):
 @pytest.mark.parametrize("kind", ["int8", "w4", "w6"])
 def test_prompt_products_match_the_32_row_products(kind, K, N):
     """Both read the same int8 planes and add the same exact int32 sums A0, A1, A2 in float32, A0 + (A1 + A2 / 254) /
-    254, with the roundings of two divisions or of two fused steps: they differ by at most one rounding of the result
-    and two of (A1 + A2 / 254) / 254, which is under a hundredth of the row's largest result on these inputs, so by
-    less than 2^-22 of that. SwiGLU: SiLU(gate) * up of the same numbers, with a float32 exp and divide (2^-20)."""
+    254, each step rounded once: bit for bit the same. SwiGLU: SiLU(gate) * up of the same numbers, with a float32 exp
+    and divide (2^-20)."""
     rng = np.random.default_rng(len(kind) + K)
     E, T = len(COUNTS), sum(COUNTS)
     fields = fields_on(_bank(kind, rng, E, N, K))
@@ -66,11 +65,53 @@ def test_prompt_products_match_the_32_row_products(kind, K, N):
     got = kernels.prompt_i8(kind, planes, scales, T, K, passes, E, fields, cb, N, order, 1)
     want = kernels.grouped_i8(kind, planes, scales, T, K, groups, work, fields, fields, cb, N, order=order2, k=1)
     got, want = got[inverse.long()].double(), want[inverse2.long()].double()  # by token
-    assert torch.all((got - want).abs() <= 2.0 ** -22 * want.abs().amax(dim=1, keepdim=True))
+    assert torch.equal(got, want)
     hidden = kernels.prompt_i8(kind, planes, scales, T, K, passes, E, fields, cb, N, order, 1, swiglu=True)
     gate, up = got[:, :N // 2], got[:, N // 2:]
     want = gate / (1 + torch.exp(-gate)) * up
     assert torch.all((hidden[inverse.long()].double() - want).abs() <= 2.0 ** -20 * (want.abs() + gate.abs() * 1e-6))
+
+
+def test_planes_meet_by_two_divisions():
+    """The int8 products' float32 epilogue, scale * (S * (A0 + (A1 + A2 / 254) / 254)) with every step rounded once, bit
+    for bit numpy's on the exact sums, in the wide and in the 32-row products."""
+    rng = np.random.default_rng(254)
+    E, N, K, T = 2, 512, 2048, 200
+    host = _bank("int8", rng, E, N, K)
+    idx = dev(np.arange(T, dtype=np.int64) % E).view(T, 1)
+    x = dev(rng.standard_normal((T, K)).astype(np.float32)).to(torch.bfloat16)
+    order, inverse, passes, planes, scales = kernels.prompt_prep_i8(idx, E, x, True)
+    order2, inverse2, groups, work, planes2, scales2 = kernels.expert_groups_prep_i8(idx, E, x, True)
+    fields = fields_on(host)
+    wide = kernels.prompt_i8("int8", planes, scales, T, K, passes, E, fields, None, N, order, 1)
+    narrow = kernels.grouped_i8("int8", planes2, scales2, T, K, groups, work, fields, fields, None, N, order=order2, k=1)
+    a = planes.view(3, T, K).double().cpu()
+    sx = scales.cpu().numpy()[:, None]
+    for e in range(E):
+        w = torch.from_numpy(host["_qdata"][e * N:(e + 1) * N]).double()
+        a0, a1, a2 = ((p[e::E] @ w.T).numpy().astype(np.float32) for p in a)  # under 2^25 in float64: exact
+        ratio = np.float32(254)
+        want = (host["scale"].reshape(-1)[e * N:(e + 1) * N].astype(np.float32)
+                * (sx[e::E] * (a0 + (a1 + a2 / ratio) / ratio)))
+        assert np.array_equal(wide[inverse.long()].cpu().numpy()[e::E], want)
+        assert np.array_equal(narrow[inverse2.long()].cpu().numpy()[e::E], want)
+
+
+@pytest.mark.parametrize("E, k, H, I", [(12, 4, 2048, 512), (5, 2, 768, 1024), (3, 1, 256, 256)])
+@pytest.mark.parametrize("kind", ["int8", "w4", "w6"])
+def test_prompt_rows_do_not_depend_on_how_many_run(kind, E, k, H, I):
+    """A row's result through the wide products, bit for bit the same rows' in prompts short enough for the 32-row ones."""
+    rng = np.random.default_rng(len(kind) + E)
+    T = 333
+    banks = [fields_on(b) for b in (_bank(kind, rng, E, 2 * I, H), _bank(kind, rng, E, H, I))]
+    cb = dev(ref.default_codebook()) if kind == "w4" else None
+    idx = dev(zipf_topk(rng, T, E, k).astype(np.int64))
+    w = dev(rng.dirichlet(np.ones(k), T).astype(np.float32))
+    x = dev(rng.standard_normal((T, H)).astype(np.float32))
+    run = lambda s: offload.resident_prefill(x[s], idx[s], w[s], banks, (2 * I, H), kind, (cb, cb), E)  # noqa: E731
+    fits = lambda n: kernels.prompt_wide_fits(kind, banks, (2 * I, H), n * k, E, H)  # noqa: E731
+    assert fits(T) and not fits(20)
+    assert torch.equal(run(slice(T)), torch.cat([run(slice(t, t + 20)) for t in range(0, T, 20)]))
 
 
 @pytest.mark.parametrize("kind", ["w4", "w6"])
