@@ -22,15 +22,18 @@ D3_INLINE uint32_t lds_address(const void* p) {
 // passing through registers. The instruction takes lds from m0: as an operand of the statement, so that the compiler
 // knows what m0 holds after it. A scalar register that a vector instruction wrote (readfirstlane) may be read by a memory
 // instruction five wait states later at the earliest: the hardware does not wait, and the compiler, which inserts an
-// s_nop 4 there before loads of its own, does not look into the statement. The compiler does not count these loads:
-// dma_wait() before the barrier that hands them to the other waves.
+// s_nop 4 there before loads of its own, does not look into the statement. A scalar instruction may read it at once, and
+// what that writes may be read at once: the base goes through an s_mov (with an s_nop 4 in its place 8192 W6 rows took
+// 0.6% longer), which is also the one wait state between setting m0 and the copy. The compiler does not count these
+// loads: dma_wait() before the barrier that hands them to the other waves.
 D3_INLINE void dma16(uint32_t lds, const void* base, uint32_t off) {
   // (both uniform already; said again for the compiler, which may keep a loop's pointers in vector registers)
   const uint64_t at = (uint64_t)base;
   const uint64_t sbase = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at) |
                          (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32;
-  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
+  uint64_t from;
+  asm volatile("s_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+               : "=&s"(from)
                : "{m0}"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(off), "s"(sbase)
                : "memory");
 }

@@ -58,12 +58,24 @@ __global__ void k(const char* const* bases, const int* lds_at) {
 """
 
 
+def _written(op):
+    """The scalar registers that an instruction (its words) writes: its first operand's."""
+    if len(op) < 2 or op[0] == "global_load_lds_dwordx4":
+        return set()
+    m = re.fullmatch(r"s\[(\d+):(\d+)\],?", op[1])
+    return set(range(int(m[1]), int(m[2]) + 1)) if m else {int(op[1][1:].rstrip(","))} if re.fullmatch(
+        r"s\d+,?", op[1]) else {"m0"} if op[1].rstrip(",") == "m0" else set()
+
+
 def test_dma16_waits_for_scalar_registers_written_by_vector_instructions(tmp_path):
-    """A base and an LDS address that come from vector registers: five wait states between the last readfirstlane and
-    the copy that reads its result (an instruction is one, s_nop n is n + 1)."""
+    """A base and an LDS address that come from vector registers: the base's two registers and m0, as the copy reads them,
+    are written by scalar instructions or five wait states before (an instruction is one, s_nop n is n + 1)."""
     lines = [line.split(";")[0].split() for line in _assembly(tmp_path, BASE_IN_VECTOR_REGISTERS).splitlines()]
     ops = [line for line in lines if line and not line[0].startswith(".") and not line[0].endswith(":")]
     copy = next(i for i, op in enumerate(ops) if op[0] == "global_load_lds_dwordx4")
-    reads = [i for i in range(copy) if ops[i][0] == "v_readfirstlane_b32"]
-    assert len(reads) >= 3
-    assert sum(int(op[1]) + 1 if op[0] == "s_nop" else 1 for op in ops[reads[-1] + 1:copy]) >= 5
+    assert sum(op[0] == "v_readfirstlane_b32" for op in ops[:copy]) >= 3
+    first, last = map(int, re.fullmatch(r"s\[(\d+):(\d+)\]", ops[copy][2]).groups())
+    for register in (first, last, "m0"):
+        writer = max(i for i in range(copy) if register in _written(ops[i]))
+        states = sum(int(op[1]) + 1 if op[0] == "s_nop" else 1 for op in ops[writer + 1:copy])
+        assert states >= (5 if ops[writer][0].startswith("v_") else 1 if register == "m0" else 0)
