@@ -5,7 +5,8 @@
 // grouped_fp8_kernel reads and widens every weight again per 32 rows. Here a workgroup runs 256 weight rows against up
 // to 96 rows: the weights lie in LDS as their e4m3 bytes, 128 columns at a time, and each wave widens its 64 rows'
 // operands as it reads them (two codes an instruction); the rows lie there as bf16, in tiles of 64 columns. A lane's
-// columns of such a tile are 16 (l >> 4) .. + 15, in two steps of 8, weights and rows alike.
+// columns of 128 are grouped_fp8_kernel's, 32 (l >> 4) .. + 31 in four steps of 8, weights and rows alike, and the planes
+// meet in its order, so that a row's float32 sums are the same however many rows run with it.
 // Measured us per layer before / here: 8192 rows, top-8 of 128 experts (FFN 768, Zipf routing) 2266 / 1331 (first bank's
 // products 546, second's 731: three planes), 2391 rows of 256 experts (FFN 512) 625 / 402.
 #include "ref_common.hpp"
@@ -48,7 +49,8 @@ D3_INLINE bf16x8 widen8(uint32_t lo, uint32_t hi) {
   return bf16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
-// A stage is 128 columns of one plane (bf16 rows as they are) or 64 columns of three; SWIGLU as wide_i8_kernel's.
+// A stage is 128 columns of one plane (bf16 rows as they are), or of three planes two of the four steps: columns 32 j +
+// 16 (s & 1) .. + 15, j < 4, of 128 in stage s. SWIGLU as wide_i8_kernel's.
 template <int PL, bool SWIGLU>
 __global__ void __launch_bounds__(WT_THREADS, 2) wide_fp8_kernel(WideF8Args a) {
   constexpr int TP = PL == 1 ? 2 : 3;      // tiles of 64 columns per row and stage: the halves, or the planes
@@ -87,14 +89,17 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_fp8_kernel(WideF8Args a) {
       for (int i = 0; i < 3; i++) p[i] = min(max(p[i], 0) / a.k_order, a.xrows - 1);
     }
 #pragma unroll
-    for (int i = 0; i < 3; i++)
-      xoff[i] = (uint32_t)p[i] * (uint32_t)(2 * K) + 16 * wt_slot(8 * ((w + 8 * i) % 12) + (lane >> 3), lane & 7);
+    for (int i = 0; i < 3; i++) {
+      const int piece = wt_slot(8 * ((w + 8 * i) % 12) + (lane >> 3), lane & 7);
+      xoff[i] = (uint32_t)p[i] * (uint32_t)(2 * K) + (PL == 1 ? 16 * piece : 64 * (piece >> 1) + 16 * (piece & 1));
+    }
   }
   auto load_rows = [&](int stage, int i) __attribute__((always_inline)) {  // copy i < COPIES of this wave
     const int n = w + 8 * i, b = n % 12, t = n / 12;
     if (n < 12 * TP && (b >> 1) < tiles)
       dma16(ldsx + (uint32_t)((stage & 1) * TP * WF_X + t * WF_X + b * 1024),
-            a.xs + (PL == 1 ? 256 * (int64_t)stage + 128 * t : t * a.plane + 128 * (int64_t)stage), xoff[i % 3]);
+            a.xs + (PL == 1 ? 256 * (int64_t)stage + 128 * t : t * a.plane + 256 * (int64_t)(stage >> 1) + 32 * (stage & 1)),
+            xoff[i % 3]);
   };
   uint32_t woff[2];
 #pragma unroll
@@ -119,11 +124,14 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_fp8_kernel(WideF8Args a) {
       for (int n = 0; n < 4; n++) acc[j][n] = part[j][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     i32x4 raw[4];
     bf16x8 b[2][PL][2];
-    int at[2];
+    int at[HALVES][2];  // step 2 h + u of the stage: piece 4 q + 2 h + u of a plane's two tiles, or 2 q + u of its one
 #pragma unroll
-    for (int u = 0; u < 2; u++) at[u] = c * 128 + 16 * wt_slot(c, 2 * q + u);
-    auto read_w = [&](int chunk, int h) __attribute__((always_inline)) {
-      const uint8_t* src = smem + (chunk & 1) * WF_W + (64 * wn) * 128 + c * 128 + 16 * wt_slot(c, 4 * h + q);
+    for (int h = 0; h < HALVES; h++)
+#pragma unroll
+      for (int u = 0; u < 2; u++)
+        at[h][u] = c * 128 + (PL == 1 ? (q >> 1) * WF_X + 16 * wt_slot(c, 4 * (q & 1) + 2 * h + u) : 16 * wt_slot(c, 2 * q + u));
+    auto read_w = [&](int chunk, int h) __attribute__((always_inline)) {  // steps 2 h and 2 h + 1 of the chunk
+      const uint8_t* src = smem + (chunk & 1) * WF_W + (64 * wn) * 128 + c * 128 + 16 * wt_slot(c, 2 * q + h);
 #pragma unroll
       for (int n = 0; n < 4; n++) raw[n] = *(const i32x4*)(src + n * 2048);
     };
@@ -132,7 +140,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_fp8_kernel(WideF8Args a) {
 #pragma unroll
       for (int t = 0; t < PL; t++)
 #pragma unroll
-        for (int u = 0; u < 2; u++) v[t][u] = *(const bf16x8*)(src + (PL == 1 ? h : t) * WF_X + at[u]);
+        for (int u = 0; u < 2; u++) v[t][u] = *(const bf16x8*)(src + (PL == 1 ? 0 : t) * WF_X + at[h][u]);
     };
     dma_wait();
     __syncthreads();
