@@ -1,12 +1,16 @@
 // The grouped products of a long prompt on A8 banks. moe_prefill.hip's grouped_kernel walks an expert's rows 16 at a
 // time past 32 weight rows held in registers, and reads every row's activations from L2 once per 32 weight rows: 48
-// times over for the first bank. That suits experts with a few rows; with hundreds, this kernel's 256 x 256 tiles read
-// both operands from L2 an eighth as often and run a wave's 64 x 128 tile from LDS (128 accumulators a lane, two waves
-// per SIMD).
+// times over for the first bank. That suits experts with a few rows; with hundreds, this kernel's tiles read both operands
+// from L2 a fourth to an eighth as often: 256 x 256 (int8), 256 weight rows x 128 (FP8) or 128 x 128 (W4, W6), a wave's 64
+// weight rows from LDS, two waves per SIMD.
 // Measured, 4096 rows, top-8 of 128 experts (FFN 768), first / second bank's products: int8 512 / 260 us before, 199 /
-// 147 here, FP8 240 / 181; the layer: int8 874 / 415, FP8 879 / 489, W4 807 / 448, W6 882 / 499 (8192 rows, Zipf
+// 147 here, FP8 240 / 181; the layer: int8 874 / 400, FP8 879 / 489, W4 807 / 459, W6 882 / 513 (8192 rows, Zipf
 // routing: int8 1703 / 698). The banks' and results' bytes take about 105 us of each int8 product at the rate a copy
 // reaches and the products 100 and 50: they overlap within a workgroup, but its first loads and its stores do not.
+// W4 and W6 as one workgroup of 256 x 128 per CU took 512 and 576 us a layer there, as 128 x 256 522 and 575; two of 128 x
+// 128 read more from L2 and cover each other's first loads, barriers and stores. (256 x 256 with the columns' groups added
+// in one run, which needs one set of accumulators, took 437 and 489, and 229 where two workgroups take 188 for 1024 rows
+// with Zipf routing.)
 #include "a8_wide.hpp"
 #include "formats.hpp"
 
@@ -14,8 +18,6 @@
 
 namespace d3 {
 namespace {
-
-constexpr int AW_W_BYTES = WT_N * 128;
 
 // acc[n] += A[n] . B, e4m3, four 16 x 16 x 128 products. One statement, as mfma_f8_chain (formats.hpp): the operands
 // keep their registers until the products have read them, and the wait states before and after cover the
@@ -40,37 +42,40 @@ D3_INLINE float add_product(float s, float a, float b) {
   return s + p;
 }
 
-// gate_up (DOWN false): a workgroup takes 128 hidden units, in LDS 32 gate rows and the same units' 32 up rows per wave.
+// gate_up (DOWN false): a workgroup's columns are half as many hidden units, in LDS 32 gate rows and the same units' 32 up
+// rows per 64.
 template <int F, bool DOWN>
-__global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
-  constexpr int TILES = a8_wide_tiles(F), AW_ROWS = 16 * TILES, AW_STAGE = AW_W_BYTES + AW_ROWS * 128;
-  constexpr int COPIES = TILES / 4;         // of 8 rows, per wave
+__global__ void __launch_bounds__(2 * a8_wide_cols(F), 2) a8_wide_kernel(A8WideArgs a) {
+  constexpr int TILES = a8_wide_tiles(F), AW_ROWS = 16 * TILES, AW_N = a8_wide_cols(F);
+  constexpr int AW_W_BYTES = AW_N * 128, AW_STAGE = AW_W_BYTES + AW_ROWS * 128;
+  constexpr int WN = AW_N / 64, WAVES = 2 * WN;  // WN waves over the weight rows (64 each), two over the pass's tiles (in turn)
+  constexpr int COPIES = 2 * TILES / WAVES;      // of 8 rows, per wave
   constexpr bool GROUPS = group_scaled(F);  // W4, W6: a scale per 128 columns, and codes to unpack
   constexpr int SRB = step_row_bytes(F);    // a stage's bytes of a weight row
   __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * AW_STAGE];
-  __shared__ __attribute__((aligned(16))) float wscale[GROUPS ? 2 : 1][WT_N];  // row scales, or a stage's group scales
+  __shared__ __attribute__((aligned(16))) float wscale[GROUPS ? 2 : 1][AW_N];  // row scales, or a stage's group scales
   __shared__ float xscale[AW_ROWS];
   __shared__ int out_row[AW_ROWS];
   const int N = a.N, K = a.K, stages = K / 128, RB = stages * SRB;
   int pass, xb;
-  wt_place(blockIdx.x, N / WT_N, pass, xb);
+  wt_place(blockIdx.x, N / AW_N, pass, xb);
   if (pass >= a.count[0]) return;
   const int4 p4 = a.passes[pass];
   const int expert = __builtin_amdgcn_readfirstlane(p4.x), first = __builtin_amdgcn_readfirstlane(p4.y),
             rows = __builtin_amdgcn_readfirstlane(p4.z), tiles = (rows + 15) / 16;
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int q = lane >> 4, c = lane & 15, wn = w & 3, wm = w >> 2;
-  const size_t n0 = (size_t)expert * N + (size_t)xb * (DOWN ? WT_N : WT_N / 2);  // the workgroup's first bank row
+  const int q = lane >> 4, c = lane & 15, wn = w % WN, wm = w / WN;
+  const size_t n0 = (size_t)expert * N + (size_t)xb * (DOWN ? AW_N : AW_N / 2);  // the workgroup's first bank row
   // the bank row, from n0, of the workgroup's row 32 * block + i, i < 32
   auto bank_row = [&](int block) { return DOWN ? 32 * block : 32 * (block >> 1) + (block & 1) * (N / 2); };
   const uint32_t lds0 = lds_address(smem);
 
-  // the pass's rows: copies of 8 rows, wave w takes copies w, w + 8, ...
+  // the pass's rows: copies of 8 rows, wave w takes copies w, w + WAVES, ...
   uint32_t xoff[COPIES];
   {
     int p[COPIES];
 #pragma unroll
-    for (int i = 0; i < COPIES; i++) p[i] = first + min(8 * (w + 8 * i) + (lane >> 3), rows - 1);
+    for (int i = 0; i < COPIES; i++) p[i] = first + min(8 * (w + WAVES * i) + (lane >> 3), rows - 1);
     if constexpr (!DOWN) {
 #pragma unroll
       for (int i = 0; i < COPIES; i++) p[i] = a.perm[p[i]];
@@ -79,22 +84,22 @@ __global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < COPIES; i++)
-      xoff[i] = (uint32_t)p[i] * (uint32_t)K + 16 * wt_slot(8 * (w + 8 * i) + (lane >> 3), lane & 7);
+      xoff[i] = (uint32_t)p[i] * (uint32_t)K + 16 * wt_slot(8 * (w + WAVES * i) + (lane >> 3), lane & 7);
     if (tid < AW_ROWS) {
       const int sp = first + min(tid, rows - 1), pair = a.perm[sp];
       out_row[tid] = pair;
       xscale[tid] = a.act_scale[DOWN ? sp : pair / a.k];
     }
-    if (!GROUPS && tid >= WT_THREADS - WT_N) {
-      const int r = tid - (WT_THREADS - WT_N);
+    if (!GROUPS && tid >= AW_N) {
+      const int r = tid - AW_N;
       wscale[0][r] = bf16_to_f32(a.s[n0 + bank_row(r >> 5) + (r & 31)]);
     }
   }
   auto load_rows = [&](int stage, int buf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < COPIES; i++)
-      if ((w + 8 * i) >> 1 < tiles)
-        dma16(lds0 + buf * AW_STAGE + AW_W_BYTES + (uint32_t)(w + 8 * i) * 1024, a.act + 128 * stage, xoff[i]);
+      if ((w + WAVES * i) >> 1 < tiles)
+        dma16(lds0 + buf * AW_STAGE + AW_W_BYTES + (uint32_t)(w + WAVES * i) * 1024, a.act + 128 * stage, xoff[i]);
   };
   const uint8_t* wwave = a.w + (n0 + bank_row(w)) * RB;
   // bytes (int8, e4m3): wave w copies rows 32 w .. 32 w + 31
@@ -118,7 +123,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
   auto load_raw = [&](int stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < RAW; i++) raw[i] = *(const i32x4*)(wwave + SRB * stage + 16 * i + doff);
-    if (tid < WT_N) raw_scale = a.s[(n0 + bank_row(tid >> 5) + (tid & 31)) * stages + stage];
+    if (tid < AW_N) raw_scale = a.s[(n0 + bank_row(tid >> 5) + (tid & 31)) * stages + stage];
   };
   auto unpack = [&](int buf) __attribute__((always_inline)) {
     uint8_t* dst = smem + buf * AW_STAGE + drow * 128;
@@ -138,7 +143,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
       *(i32x4*)(dst + 16 * wt_slot(drow, 4 * dhalf + i)) = v;
     }
     // the unpacked codes carry a factor 2^unpack_shift, taken out of the group scale (exactly)
-    if (tid < WT_N) wscale[GROUPS ? buf : 0][tid] = bf16_to_f32(raw_scale) * (1.0f / (1 << unpack_shift(F)));
+    if (tid < AW_N) wscale[GROUPS ? buf : 0][tid] = bf16_to_f32(raw_scale) * (1.0f / (1 << unpack_shift(F)));
   };
   load_rows(0, 0);
   if constexpr (GROUPS) {
@@ -157,12 +162,12 @@ __global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
     for (int j = 0; j < NT; j++)
 #pragma unroll
       for (int n = 0; n < 4; n++) acc[j][n] = Acc{0, 0, 0, 0};
-    // FP8: the sums of the K slices before this one, and the slices' length (grouped_kernel's: 4 slices of the first
-    // bank's K, 2 of the second's)
-    f32x4 sum[F == FMT_F8 ? NT : 1][4];
+    // float32 sums: those of the K slices before this one, and the slices' length (grouped_kernel's: 4 slices of the
+    // first bank's K, 2 of the second's)
+    f32x4 sum[F == FMT_I8 ? 1 : NT][4];
     const int slice = stages / (DOWN ? 2 : 4);
     int left = slice;
-    if constexpr (F == FMT_F8) {
+    if constexpr (F != FMT_I8) {
 #pragma unroll
       for (int j = 0; j < NT; j++)
 #pragma unroll
@@ -226,16 +231,20 @@ __global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
             for (int i = 0; i < 4; i++) acc[j][n][i] = fmaf((float)d[n][i], g[n][i], acc[j][n][i]);
         }
       }
-      if constexpr (F == FMT_F8) {
-        if (--left == 0) {  // the slice's sums, scaled, onto the earlier ones'
+      if constexpr (F != FMT_I8) {
+        if (--left == 0) {  // the slice's sums (FP8: scaled) onto the earlier ones'
           left = slice;
 #pragma unroll
           for (int n = 0; n < 4; n++) {
-            const f32x4 rs = *(const f32x4*)(wscale[0] + 64 * wn + 16 * n + 4 * q);
+            f32x4 rs;
+            if constexpr (F == FMT_F8) rs = *(const f32x4*)(wscale[0] + 64 * wn + 16 * n + 4 * q);
 #pragma unroll
             for (int j = 0; j < NT; j++) {
 #pragma unroll
-              for (int i = 0; i < 4; i++) sum[j][n][i] = add_product(sum[j][n][i], acc[j][n][i], rs[i]);
+              for (int i = 0; i < 4; i++) {
+                if constexpr (F == FMT_F8) sum[j][n][i] = add_product(sum[j][n][i], acc[j][n][i], rs[i]);
+                else sum[j][n][i] += acc[j][n][i];
+              }
               acc[j][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             }
           }
@@ -259,16 +268,15 @@ __global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; i++) {
             if constexpr (F == FMT_I8) v[n][i] = (float)acc[j][n][i] * rs[i] * xs;
-            else if constexpr (F == FMT_F8) v[n][i] = sum[j][n][i] * xs;
-            else v[n][i] = acc[j][n][i] * xs;
+            else v[n][i] = sum[j][n][i] * xs;
           }
         }
         if constexpr (DOWN) {
-          float* o = a.out + (size_t)out_row[r] * N + xb * WT_N + 64 * wn + 4 * q;
+          float* o = a.out + (size_t)out_row[r] * N + xb * AW_N + 64 * wn + 4 * q;
 #pragma unroll
           for (int n = 0; n < 4; n++) *(f32x4*)(o + 16 * n) = v[n];
         } else {
-          float* o = a.out + (size_t)(first + r) * (N / 2) + xb * (WT_N / 2) + 32 * wn + 4 * q;
+          float* o = a.out + (size_t)(first + r) * (N / 2) + xb * (AW_N / 2) + 32 * wn + 4 * q;
 #pragma unroll
           for (int n = 0; n < 2; n++) {
             f32x4 h;
@@ -292,10 +300,10 @@ __global__ void __launch_bounds__(WT_THREADS, 2) a8_wide_kernel(A8WideArgs a) {
 }  // namespace
 
 void launch_a8_wide(int format, bool down, const A8WideArgs& a, int cap, hipStream_t s) {
-  const dim3 grid((unsigned)(wt_places(cap) * (a.N / WT_N)));
+  const dim3 grid((unsigned)(wt_places(cap) * (a.N / a8_wide_cols(format)))), block(2 * a8_wide_cols(format));
 #define D3_AW(F)                                                                                    \
-  if (down) hipLaunchKernelGGL((a8_wide_kernel<F, true>), grid, dim3(WT_THREADS), 0, s, a);         \
-  else hipLaunchKernelGGL((a8_wide_kernel<F, false>), grid, dim3(WT_THREADS), 0, s, a);             \
+  if (down) hipLaunchKernelGGL((a8_wide_kernel<F, true>), grid, block, 0, s, a);                     \
+  else hipLaunchKernelGGL((a8_wide_kernel<F, false>), grid, block, 0, s, a);                        \
   break
   switch (format) {
     case FMT_I8: D3_AW(FMT_I8);

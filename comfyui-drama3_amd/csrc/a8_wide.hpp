@@ -1,14 +1,16 @@
-// The grouped products of a long prompt on A8 banks: 256 weight rows against up to 256 of an expert's rows per
-// workgroup (a8_wide.hip), behind d3_moe_a8_prefill.
+// The grouped products of a long prompt on A8 banks: 256 or 128 weight rows against up to 256 or 128 of an expert's rows
+// per workgroup (a8_wide.hip), behind d3_moe_a8_prefill.
 #pragma once
 #include "wide_tile.hpp"
 
 namespace d3 {
 
-// 16-row tiles of a pass. FP8 takes half as many: its float32 sums are added up as the grouped products add them, K
-// slice by K slice, so that a row's result does not depend on how many rows run with it, which takes a second set of
-// accumulators.
-__host__ __device__ constexpr int a8_wide_tiles(int format) { return format == 3 ? 8 : 16; }
+// 16-row tiles of a pass, and the weight rows of a workgroup (two threads each). int8's sums are exact; the others' float32
+// sums are added up as the grouped products add them, K slice by K slice, so that a row's result does not depend on how
+// many rows run with it. That takes a second set of accumulators, and half the rows. W4 and W6 (formats 1 and 2) also take
+// half the weight rows, which puts two workgroups on a CU.
+__host__ __device__ constexpr int a8_wide_tiles(int format) { return format == 0 ? 16 : 8; }
+__host__ __device__ constexpr int a8_wide_cols(int format) { return format == 1 || format == 2 ? 128 : 256; }
 
 struct A8WideArgs {
   const uint8_t* act;      // gate_up: the token rows [T, K]; down: the hidden rows [P, K] by sorted position

@@ -220,11 +220,11 @@ def test_prefill_experts_over_many_units(fmt, E, inter, T):
     assert counts[5] == T and counts[E - 3] >= 150
 
 
-@pytest.mark.parametrize("fmt", [formats.FMT_F8, formats.FMT_I8])
+@pytest.mark.parametrize("fmt", FMTS)
 def test_prefill_rows_independent_at_1024_rows(fmt):
     """A size-independent check past the oracle's sizes: each output row depends only on its own row (its routing,
     its pairs' hidden rows quantized per pair, each MFMA column its own dot products, its k partial outputs summed in
-    routing order), so 1024 rows at once (experts of up to ~900 pairs, split into many work units) equal, bit for
+    routing order), so 1024 rows at once (experts of up to ~900 pairs, many passes of the wide products) equal, bit for
     bit, the same rows run 16 at a time (the one-launch prep) and one at a time."""
     gate_up, down = banks(fmt, E=128, seed=11)
     gen = torch.Generator(device=DEV).manual_seed(110 + fmt)
@@ -233,7 +233,7 @@ def test_prefill_rows_independent_at_1024_rows(fmt):
     logits = zipf_logits(T, 128, seed=111 + fmt)
     out, ids, w = moe.moe_prefill(x, gate_up, down, 8, logits=logits, routing=True)
     counts = np.bincount(ids.cpu().numpy().ravel(), minlength=128)
-    assert counts.max() > 4 * 128  # the hottest expert spans five or more work units
+    assert counts.max() > 4 * 128  # the hottest expert spans three or more passes
     hot = int(np.argmax(counts))
     hot_rows = torch.nonzero((ids == hot).any(dim=1)).flatten()[:16]
     pick = torch.randperm(T, generator=torch.Generator().manual_seed(5))[:16].to(DEV)
@@ -260,11 +260,11 @@ def test_prefill_wide_products_match_oracle(fmt):
 @pytest.mark.parametrize("inter", [768, 512])
 @pytest.mark.parametrize("fmt", FMTS)
 def test_prefill_wide_products_at_tile_edges(fmt, inter):
-    """Experts with 0, 1, 15 .. 17, 255 .. 257, 300 and 530 rows, one and two per token: a row's output depends on that
-    row alone, so the wide products' rows equal the same rows run a few at a time (the grouped products, pinned on the
-    oracle) at the layer bars: their float32 sums differ in order, which can move a hidden code by one step."""
+    """Experts with 0, 1, 15 .. 17, 127 .. 129, 255 .. 257, 300 and 530 rows, one and two per token: a row's output depends
+    on that row alone, and the wide products add its sums as the grouped products (pinned on the oracle) do, so the rows
+    equal, bit for bit, the same rows run a few at a time."""
     gate_up, down = banks(fmt, inter=inter)
-    counts = [0, 1, 15, 16, 17, 31, 33, 95, 0, 255, 256, 257, 300, 530, 2, 64]
+    counts = [0, 1, 15, 16, 17, 31, 33, 95, 127, 255, 256, 257, 300, 530, 129, 128]
     rng = np.random.default_rng(fmt)
     ids = rng.permutation(np.repeat(np.arange(16), counts))
     T = len(ids)
@@ -274,9 +274,8 @@ def test_prefill_wide_products_at_tile_edges(fmt, inter):
     x = torch.randn((T, H), generator=gen, device=DEV).to(torch.bfloat16)
     for k in (1, 2):
         i, v = idx[:, :k].contiguous(), w[:, :k].contiguous()
-        got = moe.moe_prefill(x, gate_up, down, k, topk_idx=i, topk_weight=v).float().cpu().numpy()
+        got = moe.moe_prefill(x, gate_up, down, k, topk_idx=i, topk_weight=v)
         part = [moe.moe_prefill(x[t:t + 200], gate_up, down, k, topk_idx=i[t:t + 200], topk_weight=v[t:t + 200])
                 for t in range(0, T, 200)]
-        want = torch.cat(part).float().cpu().numpy()
-        assert np.all(np.isfinite(got))
-        assert_layer_close(fmt, got.astype(np.float64), want.astype(np.float64))
+        assert torch.all(torch.isfinite(got))
+        assert torch.equal(got, torch.cat(part))
