@@ -693,17 +693,22 @@ template <int F, int WIDTH> void launch_quantize(const float* src, int rows, uin
                      pair_weight, perm);
 }
 
-// From this many pairs per expert on average, the wide products (a8_wide.hip) in place of the grouped ones. Below, a
-// pass has too few rows to pay for its 256-row tile, and one workgroup per CU keeps fewer bytes on their way. Measured,
-// us per layer (grouped / wide), 128 experts with FFN 768 and 256 with FFN 512, even routing: int8 at 32 pairs 190 / 167
-// and 258 / 237 (Zipf(1.1) 195 / 200 and 277 / 257; at 37.5 218 / 207); W4 at 52 212 / 173 and 292 / 253 (Zipf 225 /
-// 217, 308 / 288; at 44 198 / 212); W6 at 52 243 / 212 and 342 / 316 (Zipf 262 / 260, 375 / 353; at 44 232 / 256): the
-// codes are read at half or three quarters the bytes, so their grouped products hold out longer.
-constexpr int A8_WIDE_PAIRS = 34, A8_WIDE_PAIRS_CODES = 52;
+// From this many pairs per expert on average, and this many in all, the wide products (a8_wide.hip) in place of the grouped
+// ones. Measured, us per layer (grouped / wide), 128 experts with FFN 768 and 256 with FFN 512, even and Zipf(1.1) routing:
+//   int8   28 pairs 188 / 174, 198 / 209, 258 / 239, 278 / 262   34 pairs 201 / 181, 214 / 214, 277 / 252, 302 / 273
+//   FP8    28 pairs 188 / 173, 199 / 199, 259 / 240, 279 / 258   34 pairs 203 / 181, 215 / 206, 278 / 252, 301 / 269
+//   W4     36 pairs 178 / 150, 183 / 175, 244 / 203, 253 / 223   W6  36 pairs 209 / 185, 219 / 215, 290 / 254, 311 / 281
+// Few experts leave the wide products a few workgroups that each walk all of K, where the grouped ones have one per 16
+// units: a shared expert (FFN 768) at 34 rows int8 26.7 / 39.3, W6 29.6 / 46.7, at 256 rows 45 / 63 and 51 / 64, at 1024
+// 55 / 71 and 60 / 72, at 2048 76 / 77 and 78 / 77, at 4096 131 / 89 and 132 / 85; 4 experts at 1024 pairs int8 57 / 73,
+// FP8 58 / 61, at 2048 90 / 78 and 90 / 67; 16 experts (FFN 512) at 1024 pairs int8 44 / 59, W4 42 / 54, at 2048 71 / 66 and
+// 67 / 59; 64 experts at 2176 pairs 112 / 105 and 96 / 92.
+constexpr int A8_WIDE_PAIRS = 34, A8_WIDE_PAIRS_IN_ALL = 2048;
 // (16-byte aligned banks: the copies to LDS need it; row offsets in 32 bits)
 bool wide_fits(const d3_moe_a8_prefill_desc& d) {
   const int64_t P = (int64_t)d.T * d.topk;
-  return P >= (int64_t)(group_scaled(d.format) ? A8_WIDE_PAIRS_CODES : A8_WIDE_PAIRS) * d.E && (((uintptr_t)d.gate_up | (uintptr_t)d.down) & 15) == 0 &&
+  return P >= std::max((int64_t)A8_WIDE_PAIRS * d.E, (int64_t)A8_WIDE_PAIRS_IN_ALL) &&
+         (((uintptr_t)d.gate_up | (uintptr_t)d.down) & 15) == 0 &&
          std::max((int64_t)d.T * d.H, P * d.I) < ((int64_t)1 << 32) - 4096;
 }
 
@@ -754,6 +759,8 @@ int64_t d3_moe_a8_prefill_workspace_bytes(int32_t T, int32_t topk, int32_t H, in
   return (int64_t)layout(T, topk, H, I, E).total;
 }
 
+int d3_moe_a8_prefill_wide(const d3_moe_a8_prefill_desc* d) { return d && wide_fits(*d); }
+
 int d3_moe_a8_prefill(const d3_moe_a8_prefill_desc* d, void* stream) {
   if (!d) return fail("d3_moe_a8_prefill: null desc");
   if (!d->x || !d->gate_up || !d->gate_up_scale || !d->down || !d->down_scale || !d->out || !d->workspace)
@@ -773,7 +780,7 @@ int d3_moe_a8_prefill(const d3_moe_a8_prefill_desc* d, void* stream) {
   // up to 16 rows: routing, x's quantization and the grouping in one launch (one workgroup). Measured on a 2048 x
   // 768, 128-expert layer, us per layer against the wide launches (then route, group and quantize): int8 66.6 / 70.8 at 7 rows, 70.2 / 74.0 at 8, 84.2 / 87.1 at 12, 97.2 / 98.6 at 16; W4A8
   // 52.1 / 56.6, 55.5 / 59.8, 64.3 / 67.3, 73.6 / 75.3.
-  const bool small = d->T <= 16 && d->topk <= 8 && d->E <= 256 && !wide_fits(*d);
+  const bool small = d->T <= 16 && d->topk <= 8 && d->E <= 256;
   if (small) {
     SmallPrepArgs sa;
     sa.logits = (const uint16_t*)d->logits;

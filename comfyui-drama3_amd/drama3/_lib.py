@@ -55,6 +55,7 @@ SIGNATURES = {
     "d3_moe_a8_noalloc_status": (c_int32, [ctypes.POINTER(c_uint32)]),
     "d3_moe_a8_prefill_workspace_bytes": (c_int64, [c_int32, c_int32, c_int32, c_int32, c_int32]),
     "d3_moe_a8_prefill": (c_int32, [ctypes.POINTER(MoeA8PrefillDesc), c_void_p]),
+    "d3_moe_a8_prefill_wide": (c_int32, [ctypes.POINTER(MoeA8PrefillDesc)]),
     "d3_gemv_a8_groups": (c_int32, [c_int32, c_void_p, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_void_p]),
     "d3_unpack_rows": (c_int32, [c_int32, c_void_p, c_int32, c_int32, c_void_p, c_void_p]),
     "d3_cvt_fp8": (c_int32, [c_void_p, c_int32, c_void_p, c_int32, c_void_p]),

@@ -291,20 +291,25 @@ def expert_groups_prep_i8(topk_idx, num_experts, x, rotate):
     return order, inverse, groups, work, planes, scales
 
 
-# From this many rows an expert on average (pairs / experts), a resident prompt's products run in wide passes
-# (96 rows against 256 weight rows per workgroup, each weight read from L2 and decoded once per pass) instead of
-# 32-row passes, which keep more weight bytes on their way while the experts have few rows. Measured us per
+# From this many rows an expert on average (pairs / experts), and this many pairs in all, a resident prompt's products run
+# in wide passes (96 rows against 256 weight rows per workgroup, each weight read from L2 and decoded once per pass)
+# instead of 32-row passes, which keep more weight bytes on their way while the experts have few rows. Measured us per
 # layer (32-row / wide), top-8 of 128 experts with FFN 768, Zipf(1.1) and even routing: int8 24 rows 192 / 199 and 164 /
 # 170, 32 rows 219 / 209 and 213 / 183; W4 24 rows 212 / 231 and 191 / 193, 32 rows 241 / 239 and 241 / 199; W6 24 rows
 # 308 / 312 and 256 / 261, 32 rows 342 / 319 and 330 / 267; fp8 24 rows 213 / 214 and 188 / 179, 32 rows 248 / 225 and
-# 230 / 193. 256 experts with FFN 512 cross between 20 and 28.
+# 230 / 193. 256 experts with FFN 512 cross between 20 and 28. Few experts leave the wide products a few workgroups that
+# each walk all of K: one expert at 512 pairs int8 37 / 64, W6 53 / 90, at 1024 54 / 68 and 78 / 93, at 2048 80 / 75 and
+# 127 / 101; 8 experts at 1024 pairs int8 56 / 66, W4 66 / 76, W6 89 / 92, fp8 65 / 67, at 2048 86 / 75, 105 / 86, 137 /
+# 101 and 103 / 76; 32 experts (FFN 512) at 960 pairs int8 55 / 59, W6 72 / 85, at 2048 76 / 70 and 108 / 94.
 PROMPT_WIDE_ROWS = 30
+PROMPT_WIDE_PAIRS = 2048
 
 
 def prompt_wide_fits(kind, banks, rows, pairs, num_experts, width):
     """Whether a resident prompt of `pairs` (row, expert) pairs over rows of `width` columns runs on prompt_i8 /
-    prompt_fp8: bank sizes in whole tiles, aligned banks, planes under 2^32 bytes, and enough rows per expert."""
-    if pairs < PROMPT_WIDE_ROWS * num_experts or num_experts > 1024:
+    prompt_fp8: bank sizes in whole tiles, aligned banks, planes under 2^32 bytes, and enough rows, per expert and in
+    all."""
+    if pairs < max(PROMPT_WIDE_ROWS * num_experts, PROMPT_WIDE_PAIRS) or num_experts > 1024:
         return False
     inner = rows[0] // 2
     weight, size = ("weight", 2) if kind == "fp8" else ("_qdata", 1)

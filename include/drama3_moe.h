@@ -147,6 +147,9 @@ typedef struct d3_moe_a8_prefill_desc {
 
 int64_t d3_moe_a8_prefill_workspace_bytes(int32_t T, int32_t topk, int32_t H, int32_t I, int32_t E);
 int d3_moe_a8_prefill(const d3_moe_a8_prefill_desc* desc, void* stream);
+/* 1 if d3_moe_a8_prefill runs this call through the wide products of long prompts, 0 if through the grouped ones (the
+ * rows' results are the same): by T, topk, E, H, I, format and the pointers' alignment alone; nothing is read. */
+int d3_moe_a8_prefill_wide(const d3_moe_a8_prefill_desc* desc);
 
 /* ---- Checks of the A8 step (no reference counterpart: they expose the fused kernels' inner operations) --------
  * d3_gemv_a8_groups: rows [R, row_bytes(K)] of a bank in `format` against C <= 16 activation rows act [C, K] (int8;

@@ -6,11 +6,13 @@ Bars as for the fused decode layer: routing ids exact and weights within one bf1
 int8 / W4A8 / W6A8, 1.5e-2 and 6e-3 for FP8 (SiLU(gate) * up in float32 with a
 fast exp before its quantization, the oracle in float64: a hidden code on a rounding boundary can differ by one step;
 FP8 adds the MFMA's inner precision)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from drama3 import formats, moe
+from drama3 import _lib, formats, moe
 from oracle import a8
 from oracle.numerics import bf16_bits_to_f32
 
@@ -48,6 +50,12 @@ def fetcher(gate_up, down):
                               b.scale[rows].contiguous().view(torch.int16).cpu().numpy().view(np.uint16))
         return cache[bank, e]
     return fetch
+
+
+def runs_wide(fmt, T, topk, E, inter):
+    """Whether T rows of an E-expert layer run through the wide products (banks as torch allocates them)."""
+    desc = _lib.MoeA8PrefillDesc(format=fmt, T=T, topk=topk, E=E, H=H, I=inter)
+    return bool(_lib.lib().d3_moe_a8_prefill_wide(ctypes.byref(desc)))
 
 
 def check(fmt, x, logits, gate_up, down, topk=8):
@@ -233,6 +241,7 @@ def test_prefill_rows_independent_at_1024_rows(fmt):
     logits = zipf_logits(T, 128, seed=111 + fmt)
     out, ids, w = moe.moe_prefill(x, gate_up, down, 8, logits=logits, routing=True)
     counts = np.bincount(ids.cpu().numpy().ravel(), minlength=128)
+    assert runs_wide(fmt, T, 8, 128, I) and not runs_wide(fmt, 16, 8, 128, I)
     assert counts.max() > 4 * 128  # the hottest expert spans three or more passes
     hot = int(np.argmax(counts))
     hot_rows = torch.nonzero((ids == hot).any(dim=1)).flatten()[:16]
@@ -249,11 +258,12 @@ def test_prefill_rows_independent_at_1024_rows(fmt):
 
 @pytest.mark.parametrize("fmt", FMTS)
 def test_prefill_wide_products_match_oracle(fmt):
-    """Enough pairs per expert (54 on average) for the wide products: against the oracle at the layer bars."""
+    """Enough pairs (2072, 129.5 per expert on average) for the wide products: against the oracle at the layer bars."""
     gate_up, down = banks(fmt)
     gen = torch.Generator(device=DEV).manual_seed(60 + fmt)
-    x = torch.randn((108, H), generator=gen, device=DEV).to(torch.bfloat16)
-    logits = torch.randn((108, 16), generator=gen, device=DEV).to(torch.bfloat16)
+    x = torch.randn((259, H), generator=gen, device=DEV).to(torch.bfloat16)
+    logits = torch.randn((259, 16), generator=gen, device=DEV).to(torch.bfloat16)
+    assert runs_wide(fmt, 259, 8, 16, I)
     check(fmt, x, logits, gate_up, down)
 
 
@@ -273,6 +283,7 @@ def test_prefill_wide_products_at_tile_edges(fmt, inter):
     w = torch.rand((T, 2), generator=gen, device=DEV)
     x = torch.randn((T, H), generator=gen, device=DEV).to(torch.bfloat16)
     for k in (1, 2):
+        assert runs_wide(fmt, T, k, 16, inter) and not runs_wide(fmt, 200, k, 16, inter)
         i, v = idx[:, :k].contiguous(), w[:, :k].contiguous()
         got = moe.moe_prefill(x, gate_up, down, k, topk_idx=i, topk_weight=v)
         part = [moe.moe_prefill(x[t:t + 200], gate_up, down, k, topk_idx=i[t:t + 200], topk_weight=v[t:t + 200])
