@@ -704,11 +704,11 @@ template <int F, int WIDTH> void launch_quantize(const float* src, int rows, uin
 // FP8 58 / 61, at 2048 90 / 78 and 90 / 67; 16 experts (FFN 512) at 1024 pairs int8 44 / 59, W4 42 / 54, at 2048 71 / 66 and
 // 67 / 59; 64 experts at 2176 pairs 112 / 105 and 96 / 92.
 constexpr int A8_WIDE_PAIRS = 34, A8_WIDE_PAIRS_IN_ALL = 2048;
-// (16-byte aligned banks: the copies to LDS need it; row offsets in 32 bits)
+// (16-byte aligned banks and workspace, where the quantized rows lie: the copies to LDS need it; row offsets in 32 bits)
 bool wide_fits(const d3_moe_a8_prefill_desc& d) {
   const int64_t P = (int64_t)d.T * d.topk;
   return P >= std::max((int64_t)A8_WIDE_PAIRS * d.E, (int64_t)A8_WIDE_PAIRS_IN_ALL) &&
-         (((uintptr_t)d.gate_up | (uintptr_t)d.down) & 15) == 0 &&
+         (((uintptr_t)d.gate_up | (uintptr_t)d.down | (uintptr_t)d.workspace) & 15) == 0 &&
          std::max((int64_t)d.T * d.H, P * d.I) < ((int64_t)1 << 32) - 4096;
 }
 

@@ -26,7 +26,8 @@ def test_a8_prefill_rule(fmt):
         assert not a8_wide(fmt, *call), call
     for call in LONG:
         assert a8_wide(fmt, *call), call
-        assert not a8_wide(fmt, *call, gate_up=1024 + 8) and not a8_wide(fmt, *call, down=1024 + 1), call
+        for pointer in ("gate_up", "down", "workspace"):
+            assert a8_wide(fmt, *call, **{pointer: 1024 + 16}) and not a8_wide(fmt, *call, **{pointer: 1024 + 8}), call
     assert not a8_wide(fmt, 2 ** 20, 8, 128, 768)  # hidden rows past 2^32 bytes
 
 
