@@ -1,13 +1,9 @@
-// What the kernels of the reference's own formats share: the 4-bit codes' tables, the int8 planes' ratio and the row
-// of the planes that a prompt's pair reads.
+// What the kernels of the reference's own formats share: the 4-bit codes' tables, the int8 planes' ratio and sum, SiLU(gate)
+// * up, and the row of the planes that a prompt's pair reads.
 #pragma once
 #include "common.hpp"
 
 namespace d3 {
-
-template <int CTRL> D3_INLINE float dpp_f32(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
 
 // W4 through tables: a 16-column group's codes all share one e4m3 scale byte, so the int8-grid values of the 16 codes at
 // each of the 256 scale bytes make a 4 KB table (decode_group's own arithmetic, entry by entry), kept in LDS as bytes
@@ -73,9 +69,11 @@ D3_INLINE i32x4 w4_group_i8(uint32_t lo, uint32_t hi, i32x4 t) {
 }
 
 // The row of the planes that row p of the passes reads: p itself, or with `order` x's row order[p] / k (the rows of
-// a prompt's pairs taken from its token rows, so no gathered copy is made), kept within the planes' xrows rows.
+// a prompt's pairs taken from its token rows, so no gathered copy is made), kept within the planes' xrows rows. (The wide
+// products request all their pairs before they use one: pair_row alone.)
+D3_INLINE int pair_row(int64_t pair, int k, int xrows) { return min(max((int)pair, 0) / k, xrows - 1); }
 D3_INLINE size_t plane_row(const int64_t* order, int k, int xrows, int p) {
-  return order ? (size_t)min(max((int)order[p], 0) / k, xrows - 1) : (size_t)p;
+  return order ? (size_t)pair_row(order[p], k, xrows) : (size_t)p;
 }
 
 }  // namespace d3

@@ -117,8 +117,8 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_i8_kernel(WideArgs a) {
       for (int i = 0; i < 3; i++) p[i] = (int)a.order[p[i]];
       own = (int)a.order[own];
 #pragma unroll
-      for (int i = 0; i < 3; i++) p[i] = min(max(p[i], 0) / a.k_order, a.xrows - 1);
-      own = min(max(own, 0) / a.k_order, a.xrows - 1);
+      for (int i = 0; i < 3; i++) p[i] = pair_row(p[i], a.k_order, a.xrows);
+      own = pair_row(own, a.k_order, a.xrows);
     }
 #pragma unroll
     for (int i = 0; i < 3; i++)

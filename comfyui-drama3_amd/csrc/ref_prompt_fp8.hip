@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(WT_THREADS, 2) wide_fp8_kernel(WideF8Args a) {
 #pragma unroll
       for (int i = 0; i < 3; i++) p[i] = (int)a.order[p[i]];
 #pragma unroll
-      for (int i = 0; i < 3; i++) p[i] = min(max(p[i], 0) / a.k_order, a.xrows - 1);
+      for (int i = 0; i < 3; i++) p[i] = pair_row(p[i], a.k_order, a.xrows);
     }
 #pragma unroll
     for (int i = 0; i < 3; i++) {
