@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(256) rotate_kernel(const void* x, int K, float
       const f32x4 gt = *(const f32x4*)(f + c0), up = *(const f32x4*)(f + K + c0);
       const float gg[4] = {gt.x, gt.y, gt.z, gt.w}, uu[4] = {up.x, up.y, up.z, up.w};
 #pragma unroll
-      for (int j = 0; j < 4; j++) v[j] = gg[j] / (1.0f + __expf(-gg[j])) * uu[j];
+      for (int j = 0; j < 4; j++) v[j] = silu_up(gg[j], uu[j]);
     }
     fwht256(v);
     *(f32x4*)(out + (size_t)row * K + c0) = f32x4{v[0], v[1], v[2], v[3]};
