@@ -608,8 +608,12 @@ def run_resident_prompt(args, fmt, device):
               "us_per_layer": round(ms * 1e3 / (args.steps * L), 2),
               "mfma_ops_per_s_e12": round(flops * L * args.steps / (ms * 1e-3) / 1e12, 2),
               "mfma_type": "bf16" if args.format == "fp8" else "int8"}
+    kind, banks, _ = layers[0]
+    wide = kernels.prompt_wide_fits(kind, banks, rows, T * TOPK, E, H)
+    products = ("wide_fp8_kernel" if kind == "fp8" else "wide_i8_kernel") if wide else (
+        "grouped_fp8_kernel" if kind == "fp8" else "grouped_i8_kernel")
     return (ms, step_bytes * args.steps, args.steps * L, args.steps * T, config,
-            "route + resident_prefill (d3::grouped_i8_kernel / grouped_fp8_kernel per bank, 7 launches)", None)
+            f"route + resident_prefill (d3::{products} per bank)", None)
 
 
 def run_resident(args, fmt, device):

@@ -3,9 +3,9 @@
 // times over for the first bank. That suits experts with a few rows; with hundreds, this kernel's tiles read both operands
 // from L2 a fourth to an eighth as often: 256 x 256 (int8), 256 weight rows x 128 (FP8) or 128 x 128 (W4, W6), a wave's 64
 // weight rows from LDS, two waves per SIMD.
-// Measured, 4096 rows, top-8 of 128 experts (FFN 768), first / second bank's products: int8 512 / 260 us before, 199 /
-// 147 here, FP8 240 / 181; the layer: int8 874 / 400, FP8 879 / 489, W4 807 / 459, W6 882 / 513 (8192 rows, Zipf
-// routing: int8 1703 / 698). The banks' and results' bytes take about 105 us of each int8 product at the rate a copy
+// Measured, 4096 rows, top-8 of 128 experts (FFN 768), first / second bank's products in a kernel trace: int8 511 / 262 us
+// before, 182 / 140 here, FP8 234 / 174, W4 230 / 161, W6 261 / 178; the layer untraced: int8 874 / 400, FP8 879 / 485, W4
+// 807 / 459, W6 882 / 513 (8192 rows, Zipf routing: int8 1703 / 706). The banks' and results' bytes take about 105 us of each int8 product at the rate a copy
 // reaches and the products 100 and 50: they overlap within a workgroup, but its first loads and its stores do not.
 // W4 and W6 as one workgroup of 256 x 128 per CU took 512 and 576 us a layer there, as 128 x 256 522 and 575; two of 128 x
 // 128 read more from L2 and cover each other's first loads, barriers and stores. (256 x 256 with the columns' groups added

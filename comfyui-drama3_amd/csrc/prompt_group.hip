@@ -1,7 +1,5 @@
 // A long prompt's pairs grouped by expert (offload.py:140-143's sort and counts), see prompt_group.hpp: two launches,
-// the blocks' counts and the dealing. Measured for
-// 32768 and 65536 pairs of 128 experts: 11 and 13 us on A8 banks (one workgroup: 36 and 57), 8 us after the counts that
-// ride with the rows' planes on the reference's (19128 pairs of 256 experts: 31 us in one workgroup).
+// the blocks' counts and the dealing.
 #include "prompt_group.hpp"
 
 namespace d3 {

@@ -6,11 +6,11 @@
 // weight rows read all of the pass's planes from LDS; the matrix cores were busy 10 to 20% of the time. Here a
 // workgroup runs 256 weight rows against up to 96 rows (288 plane rows), a wave 64 x 48 (x 3 planes): 144 accumulators
 // a lane, which still leaves two waves per SIMD, and a weight is read from L2 and decoded once per 96 rows.
-// Measured, 8192 rows, top-8 of 128 experts (FFN 768, Zipf routing), both banks' products before / after: int8 about
-// 1700 / 1000 us, W4 2200 / 1200, W6 3330 / 1640 (the layer: 1983 / 1235, 2430 / 1430, 3378 / 1675). int8's products
-// alone (no copies, no stores) take 417 us of the first bank's 600 and the copies alone 364: what is left is L2
-// misses that one stage ahead does not cover, and the stores (dn: 537 MB of float32). W6 adds its decoding, about 4
-// vector instructions a code and pass.
+// Measured, 8192 rows, top-8 of 128 experts (FFN 768, Zipf routing), both banks' products in a kernel trace, 32-row / here:
+// int8 1849 / 1148 us, W4 2361 / 1383, W6 3317 / 1640; the layer untraced 1983 / 1253, 2430 / 1455, 3378 / 1695. int8's
+// products alone (no copies, no stores) take 417 us of the first bank's 632 and the copies alone 364: what is left is L2
+// misses that one stage ahead does not cover, and the stores (dn: 537 MB of float32). W6 adds its decoding, about 85
+// vector instructions per 16 codes and pass. (The planes' sums by divisions, as the 32-row products', take 1% of a layer.)
 #include "ref_common.hpp"
 #include "wide_tile.hpp"
 #include "../../include/drama3_moe.h"

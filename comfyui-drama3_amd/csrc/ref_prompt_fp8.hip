@@ -7,8 +7,9 @@
 // operands as it reads them (two codes an instruction); the rows lie there as bf16, in tiles of 64 columns. A lane's
 // columns of 128 are grouped_fp8_kernel's, 32 (l >> 4) .. + 31 in four steps of 8, weights and rows alike, and the planes
 // meet in its order, so that a row's float32 sums are the same however many rows run with it.
-// Measured us per layer before / here: 8192 rows, top-8 of 128 experts (FFN 768, Zipf routing) 2266 / 1331 (first bank's
-// products 546, second's 731: three planes), 2391 rows of 256 experts (FFN 512) 625 / 402.
+// Measured us per layer, 32-row / here: 8192 rows, top-8 of 128 experts (FFN 768, Zipf routing) 2266 / 1352 (in a kernel
+// trace the first bank's products 1196 / 560, the second's, three planes, 966 / 752), 2391 rows of 256 experts (FFN 512)
+// 625 / 414. (With the columns in memory order, whole 128-byte lines a copy, 1331 and 408: other sums at other lengths.)
 #include "ref_common.hpp"
 #include "wide_tile.hpp"
 #include "../../include/drama3_moe.h"
