@@ -1,16 +1,17 @@
 // The grouped products of a long prompt on A8 banks. moe_prefill.hip's grouped_kernel walks an expert's rows 16 at a
 // time past 32 weight rows held in registers, and reads every row's activations from L2 once per 32 weight rows: 48
-// times over for the first bank. That suits experts with a few rows; with hundreds, this kernel's tiles read both operands
-// from L2 a fourth to an eighth as often: 256 x 256 (int8), 256 weight rows x 128 (FP8) or 128 x 128 (W4, W6), a wave's 64
-// weight rows from LDS, two waves per SIMD.
-// Measured, 4096 rows, top-8 of 128 experts (FFN 768), first / second bank's products in a kernel trace: int8 511 / 262 us
-// before, 182 / 140 here, FP8 234 / 174, W4 230 / 161, W6 261 / 178; the layer untraced: int8 874 / 400, FP8 879 / 485, W4
-// 807 / 459, W6 882 / 513 (8192 rows, Zipf routing: int8 1703 / 706). The banks' and results' bytes take about 105 us of each int8 product at the rate a copy
-// reaches and the products 100 and 50: they overlap within a workgroup, but its first loads and its stores do not.
-// W4 and W6 as one workgroup of 256 x 128 per CU took 512 and 576 us a layer there, as 128 x 256 522 and 575; two of 128 x
-// 128 read more from L2 and cover each other's first loads, barriers and stores. (256 x 256 with the columns' groups added
-// in one run, which needs one set of accumulators, took 437 and 489, and 229 where two workgroups take 188 for 1024 rows
-// with Zipf routing.)
+// times over for the first bank. That suits experts with a few rows; with hundreds, this kernel's tiles read both
+// operands from L2 a fourth to an eighth as often: 256 x 256 (int8), 256 weight rows x 128 (FP8) or 128 x 128 (W4,
+// W6), a wave's 64 weight rows from LDS, two waves per SIMD.
+// Measured, 4096 rows, top-8 of 128 experts (FFN 768), first / second bank's products in a kernel trace: int8 511 /
+// 262 us before, 182 / 140 here, FP8 234 / 174, W4 230 / 161, W6 261 / 178; the layer untraced: int8 874 / 400, FP8
+// 879 / 485, W4 807 / 459, W6 882 / 513 (8192 rows, Zipf routing: int8 1703 / 706). The banks' and results' bytes take
+// about 105 us of each int8 product at the rate a copy reaches and the products 100 and 50: they overlap within a
+// workgroup, but its first loads and its stores do not.
+// W4 and W6 as one workgroup of 256 x 128 per CU took 512 and 576 us a layer there, as 128 x 256 522 and 575; two of
+// 128 x 128 read more from L2 and cover each other's first loads, barriers and stores. (256 x 256 with the columns'
+// groups added in one run, which needs one set of accumulators, took 437 and 489, and 229 where two workgroups take
+// 188 for 1024 rows with Zipf routing.)
 #include "a8_wide.hpp"
 #include "formats.hpp"
 
@@ -48,7 +49,7 @@ template <int F, bool DOWN>
 __global__ void __launch_bounds__(2 * a8_wide_cols(F), 2) a8_wide_kernel(A8WideArgs a) {
   constexpr int TILES = a8_wide_tiles(F), AW_ROWS = 16 * TILES, AW_N = a8_wide_cols(F);
   constexpr int AW_W_BYTES = AW_N * 128, AW_STAGE = AW_W_BYTES + AW_ROWS * 128;
-  constexpr int WN = AW_N / 64, WAVES = 2 * WN;  // WN waves over the weight rows (64 each), two over the pass's tiles (in turn)
+  constexpr int WN = AW_N / 64, WAVES = 2 * WN;  // WN over the weight rows (64 each), two over the pass's tiles (in turn)
   constexpr int COPIES = 2 * TILES / WAVES;      // of 8 rows, per wave
   constexpr bool GROUPS = group_scaled(F);  // W4, W6: a scale per 128 columns, and codes to unpack
   constexpr int SRB = step_row_bytes(F);    // a stage's bytes of a weight row
